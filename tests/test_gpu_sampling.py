@@ -101,3 +101,42 @@ def test_bad_temperature_is_an_error(pkg, dev):
     x = torch.zeros(2, 10, device=dev)
     with pytest.raises(RuntimeError, match="temperature"):
         pkg.sample_rows(x, float("nan"), 1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("V,pad", [(1, 0), (1023, 0), (1024, 4), (1028, 1), (8196, 0), (60011, 5)])
+def test_sample_rows_skipped_candidates_change_nothing(pkg, dev, dtype, V, pad):
+    """The kernel evaluates only candidates whose bound passes the best seen: at the edges of its
+    groups of four, threads and chunks, in aligned and unaligned rows, and with masked (-inf),
+    infinite, NaN and equal logits, the pick is that of all candidates."""
+    print(f"case sampling bounds V={V} pad={pad} {dtype}", flush=True)
+    M, T, seed = 9, 0.7, 31
+    g = torch.Generator().manual_seed(V)
+    full = (torch.randn(M, V + pad, generator=g) * 4).to(dtype)
+    x = full[:, :V]
+    x[1] = 0.25                                   # equal logits: the noise alone decides
+    x[2] = float("-inf")                          # all masked
+    x[3] = float("-inf")
+    x[3, V // 2] = -3.0                           # one candidate left
+    x[4, torch.rand(V, generator=g) < 0.9] = float("-inf")
+    x[5, V - 1] = x[5, V // 3] = float("inf")     # the lowest of two infinities
+    x[6, V - 1] = x[6, V // 2] = float("nan")     # the first NaN
+    x[7] *= 40.0                                  # float16: quotients near its largest value
+    full = full.to(dev)
+    ids, score = pkg.sample_rows(full[:, :V], T, seed)
+    torch.cuda.synchronize()
+    finite = [0, 1, 3, 4, 7, 8]
+    name = _NAMES[dtype]
+    s = S.perturbed_scores(x.float().numpy(), T, seed, 0, name)
+    ids, score = ids.cpu().numpy(), score.cpu().numpy()
+    for m in finite:
+        if not np.isfinite(s[m]).any():           # V small enough that row 4 is all masked
+            continue
+        best = s[m].max()
+        # the two logarithms of device and oracle differ by a few units in the last place of terms up to 17
+        tol = 1e-5 * max(1.0, abs(best))
+        assert s[m, ids[m]] >= best - tol, (m, ids[m], s[m].argmax())
+        np.testing.assert_allclose(score[m], s[m, ids[m]], rtol=4e-6, atol=4e-6)
+    assert ids[2] == 0 and score[2] == -np.inf
+    assert ids[5] == V // 3 and score[5] == np.inf
+    assert ids[6] == V // 2 and np.isnan(score[6])
