@@ -1,10 +1,12 @@
 // Host side of the fused combine + argmax: workspace layout and dispatch to
 // the per-dtype instantiations of the GEMV kernel (fused_argmax_gemv.h, few
-// rows) and of the MFMA-tiled kernel (fused_argmax_tiled.h, many rows).
+// rows), of the 17-to-64-row streaming kernel (fused_argmax_rows.h) and of the
+// MFMA-tiled kernel (fused_argmax_tiled.h, many rows).
 #include <algorithm>
 
 #include "fused_argmax_fp8.h"
 #include "fused_argmax_gemv.h"
+#include "fused_argmax_rows.h"
 #include "fused_argmax_tiled.h"
 #include "fused_argmax_tiled8.h"
 #include "lowrank_decode.h"
@@ -36,6 +38,26 @@ bool tiled_eligible(const ArgmaxArgs& a) {
         if ((reinterpret_cast<uintptr_t>(a.prior) & 3) != 0 || (pb == 2 && (a.V & 1) != 0)) return false;
     }
     return (reinterpret_cast<uintptr_t>(a.rank) & 15) == 0 && a.ldrank % 8 == 0;
+}
+
+// Rows from which the streaming kernel that shares each tile of B among several
+// groups of 16 rows takes over from the 16-row GEMV kernel: that one reads B
+// once per group, so two groups already cost it a second pass (24 rows, r = 256,
+// V = 151936, per step of a rollout: 43.9 us, 38.0 us here).
+constexpr int kRowsMinRows = 17;
+
+bool rows_eligible(const ArgmaxArgs& a, int prior_kind) {
+    return a.M >= kRowsMinRows && rows_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+}
+
+// Four-element loads of base and prior: aligned rows of whole quads, and byte
+// offsets into base that fit 32 bits.
+bool rows_vec(const ArgmaxArgs& a) {
+    const int eb = base_elem_bytes(a.base_dtype);
+    if (a.V % 4 != 0 || a.ldbase % 4 != 0 || (reinterpret_cast<uintptr_t>(a.base) % (4 * eb)) != 0) return false;
+    if (a.prior != nullptr && (reinterpret_cast<uintptr_t>(a.prior) % (4 * base_elem_bytes(a.prior_dtype))) != 0)
+        return false;
+    return ((int64_t)(a.M - 1) * a.ldbase + a.V) * eb < ((int64_t)1 << 32);
 }
 
 }  // namespace
@@ -94,6 +116,12 @@ hipError_t launch_fused_argmax(const ArgmaxArgs& a, void* ws, size_t data_off, h
     ka.keys = reinterpret_cast<unsigned long long*>(w + kKeysOff);
     // one 128-byte line per row while the rows fit the key area, else packed
     ka.key_stride = (int64_t)a.M * 128 <= (int64_t)(kCtrlBytes - kKeysOff) ? 16 : 1;
+    if (rows_eligible(a, pk)) {
+        const bool vec = rows_vec(a);
+        if (a.base_dtype == 1) return launch_rows_bf16(ka, a.b_packed, pk, vec, s);
+        if (a.base_dtype == 2) return launch_rows_f16(ka, a.b_packed, pk, vec, s);
+        return launch_rows_f32(ka, a.b_packed, pk, vec, s);
+    }
     if (a.base_dtype == 1) return launch_gemv_bf16(ka, a.b_packed, pk, s);
     if (a.base_dtype == 2) return launch_gemv_f16(ka, a.b_packed, pk, s);
     return launch_gemv_f32(ka, a.b_packed, pk, s);

@@ -1,0 +1,278 @@
+// Fused low-rank LM-head combine + vocabulary argmax for 17 to 64 rows per
+// pass over B: the streaming kernel between the 16-row GEMV kernel and the
+// MFMA-tiled one, and the general one for more rows wherever the tiled kernel
+// does not apply (row-major B, unaligned rows, a rank it does not take).
+//
+// Semantics as the GEMV kernel (code/kernel/dels.py:42-138):
+//     s[m, v] = fma(-beta_m, prior[v], fma(fp32(rank_m . B[v]), alpha_m, base[m, v]))
+// and per row the lowest v attaining max_v s[m, v].  The contraction sums the
+// same MFMA K steps in the same order, so scores equal the GEMV kernel's bit
+// for bit.
+//
+// Bound by streaming B from HBM once: a workgroup keeps the rank operand of RG
+// groups of 16 rows in registers (RG * r / 8 VGPRs: 256 of the 512 a wave has at
+// one wave per SIMD, for 64 rows at r = 512), so that every 16-row vocabulary
+// tile that a wave loads serves all of them, instead of being read again for
+// every 16 rows.  The tile is the MFMA's A operand and the rank its B operand:
+// lane l ends with row l % 16 of each group and the four consecutive columns
+// 4 (l / 16) .. + 3, so that a lane's base logits are one 8- or 16-byte load per
+// group, its prior values one load for all groups, and the running argmax takes
+// one (score, index) pair per group.  Streaming as in the GEMV kernel: tiles
+// walked wave-strided through two register sets, refills unconditional.
+// 40 rows, r = 512, V = 151936, bf16 base logits, whole step with its 12 us rank
+// projection: 115 us with the GEMV kernel (B read three times), 49 us here.
+#pragma once
+
+#include "fused_argmax_gemv.h"
+#include "fused_argmax_tiled.h"
+
+namespace dels {
+
+namespace rows {
+
+constexpr int kThreads = 256;
+
+// Values a lane takes from a row per tile: four consecutive ones.  VEC: as one
+// load (two words of 16-bit values, four of fp32), else four element loads.
+template <typename T, bool VEC>
+constexpr int quad_words() { return VEC && sizeof(T) == 2 ? 2 : 4; }
+
+// Row offsets (bytes) fit 32 bits with VEC, so that a row costs one register.
+template <bool VEC>
+using RowOff = typename std::conditional<VEC, uint32_t, int64_t>::type;
+
+template <typename T, bool VEC>
+__device__ __forceinline__ void load_quad(const void* base, RowOff<VEC> row, int v, int V,
+                                          uint32_t (&w)[quad_words<T, VEC>()]) {
+    const char* p = static_cast<const char*>(base);
+    if constexpr (VEC) {
+        const uint32_t o = row + (uint32_t)min(v, V - 4) * (uint32_t)sizeof(T);   // V a multiple of 4: whole quads
+        if constexpr (sizeof(T) == 2) {
+            const u32x2 x = __builtin_nontemporal_load(reinterpret_cast<const u32x2*>(p + o));
+            w[0] = x[0]; w[1] = x[1];
+        } else {
+            const u32x4 x = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + o));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) w[q] = x[q];
+        }
+    } else {
+        const T* r = reinterpret_cast<const T*>(p + row);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = load_raw(r + min(v + q, V - 1));
+    }
+}
+
+// Value q of a quad, widened.
+template <typename T, bool VEC>
+__device__ __forceinline__ float quad_at(const uint32_t (&w)[quad_words<T, VEC>()], int q) {
+    if constexpr (VEC && sizeof(T) == 2) return tiled::half_at<T>(w[q >> 1], q & 1);
+    else return widen_raw<T>(w[q]);
+}
+
+// Row groups per workgroup above 32 rows: 4, or 3 where the four words of base
+// logits per group and tile (fp32, or unaligned rows) leave no registers for
+// the fourth group's 64 at r = 512.
+template <int KSTEPS, typename BaseT, bool VEC>
+constexpr int max_groups() { return KSTEPS == 16 && quad_words<BaseT, VEC>() == 4 ? 3 : 4; }
+
+}  // namespace rows
+
+// Ranks the kernel takes: whole MFMA K steps, no masked operands.
+inline bool rows_rank_ok(int r) { return r == 128 || r == 256 || r == 512; }
+
+template <int RG, int KSTEPS, typename BaseT, typename PriorT, bool VEC>
+struct RowsTile {
+    bf16x8 b[KSTEPS];
+    uint32_t base[RG][rows::quad_words<BaseT, VEC>()];
+    uint32_t prior[rows::quad_words<PriorT, VEC>()];
+};
+
+// HAS_PRIOR false: the prior term is absent (PriorT is then BaseT and unused).
+template <int RG, int KSTEPS, bool ROWMAJOR, typename BaseT, typename PriorT, bool VEC, bool HAS_PRIOR>
+__global__ __launch_bounds__(rows::kThreads, 1) void fused_argmax_rows_kernel(ArgmaxKArgs a) {
+#pragma clang fp contract(off)
+    using namespace rows;
+    constexpr int kRows = 16 * RG;
+    __shared__ float s_val[4][kRows];
+    __shared__ int s_idx[4][kRows];
+    __shared__ int s_last;
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar loop control
+    const int col = lane & 15;     // row of the lane within each group
+    const int kg = lane >> 4;      // K octet of the operands / quad of columns of the results
+    const int m0 = blockIdx.y * kRows;
+
+    // Rank operands of the groups' rows, resident for the whole kernel; rows
+    // past M repeat row 0 (their results are not written).
+    bf16x8 ra[RG][KSTEPS];
+    float al[RG], nbe[RG], best[RG];
+    int bidx[RG];
+    bool use_prior[RG];
+    RowOff<VEC> brow[RG];
+#pragma unroll
+    for (int g = 0; g < RG; ++g) {
+        const int m = m0 + 16 * g + col;
+        const int mc = m < a.M ? m : 0;
+        const uint16_t* rp = a.rank + rank_row_of(a.rank_rows, a.rank_rows_stride, a.rank_rows_count, mc) * a.ldrank;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) ra[g][s] = load_bf16x8(rp + s * 32 + kg * 8);
+        al[g] = a.alpha[(int64_t)mc * a.alpha_stride];
+        const float be = a.beta[(int64_t)mc * a.beta_stride];
+        nbe[g] = -be;
+        use_prior[g] = HAS_PRIOR && be != 0.f;
+        brow[g] = (RowOff<VEC>)((int64_t)mc * a.ldbase * (int64_t)sizeof(BaseT));
+        best[g] = -__builtin_inff();
+        bidx[g] = INT_MAX;
+    }
+
+    using Tile = RowsTile<RG, KSTEPS, BaseT, PriorT, VEC>;
+    auto load = [&](int t, Tile& tr) {
+        // ROWMAJOR: the lane's K octets of vocabulary row t * 16 + col; else MFMA-16 blocks
+        const uint16_t* bp = ROWMAJOR ? a.B + (int64_t)min(t * 16 + col, a.V - 1) * a.ldb + kg * 8
+                                      : a.B + (int64_t)t * (KSTEPS * 512) + lane * 8;
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) tr.b[s] = load_bf16x8_nt(bp + s * (ROWMAJOR ? 32 : 512));
+        const int v = t * 16 + 4 * kg;
+#pragma unroll
+        for (int g = 0; g < RG; ++g) load_quad<BaseT, VEC>(a.base, brow[g], v, a.V, tr.base[g]);
+        if constexpr (HAS_PRIOR) load_quad<PriorT, VEC>(a.prior, 0, v, a.V, tr.prior);
+    };
+    auto consume = [&](const Tile& tr, int t) {
+        f32x4 acc[RG];
+#pragma unroll
+        for (int g = 0; g < RG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int g = 0; g < RG; ++g)
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr.b[s], ra[g][s], acc[g], 0, 0, 0);
+        const int v = t * 16 + 4 * kg;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool in = v + q < a.V;
+            float pv = 0.f;
+            if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
+#pragma unroll
+            for (int g = 0; g < RG; ++g) {
+                float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT, VEC>(tr.base[g], q));
+                if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
+                // a lane's candidates arrive in increasing column order: strict ">" keeps the lowest index
+                const bool take = in & (sc > best[g]);
+                best[g] = take ? sc : best[g];
+                bidx[g] = take ? v + q : bidx[g];
+            }
+        }
+    };
+
+    // the tiles t + k * nwaves, k < cnt, through two register sets (see the GEMV kernel)
+    const int ntiles = (a.V + 15) >> 4;
+    const int nwaves = gridDim.x * 4;
+    const int t = blockIdx.x * 4 + wave;
+    const int cnt = t < ntiles ? (ntiles - 1 - t) / nwaves + 1 : 0;
+    Tile tr0, tr1;
+    if (cnt > 0) load(t, tr0);
+    if (cnt > 1) load(t + nwaves, tr1);
+    int k = 0;
+    for (; k + 4 <= cnt; k += 2) {
+        consume(tr0, t + k * nwaves);
+        load(t + (k + 2) * nwaves, tr0);
+        consume(tr1, t + (k + 1) * nwaves);
+        load(t + (k + 3) * nwaves, tr1);
+    }
+    if (k < cnt) consume(tr0, t + k * nwaves);
+    if (k + 2 < cnt) load(t + (k + 2) * nwaves, tr0);
+    if (k + 1 < cnt) consume(tr1, t + (k + 1) * nwaves);
+    if (k + 2 < cnt) consume(tr0, t + (k + 2) * nwaves);
+
+    // each row's best over the four quads of columns, then over the waves
+#pragma unroll
+    for (int g = 0; g < RG; ++g) {
+#pragma unroll
+        for (int off = 16; off < 64; off <<= 1) {
+            const float ov = __shfl_xor(best[g], off, 64);
+            const int oi = __shfl_xor(bidx[g], off, 64);
+            if (argmax_better(ov, oi, best[g], bidx[g])) {
+                best[g] = ov;
+                bidx[g] = oi;
+            }
+        }
+        if (kg == 0) {
+            s_val[wave][16 * g + col] = best[g];
+            s_idx[wave][16 * g + col] = bidx[g];
+        }
+    }
+    __syncthreads();
+    int fin_m[1] = {-1};
+    unsigned long long fin_key[1] = {0ull};
+    if (threadIdx.x < kRows) {
+        const int mi = threadIdx.x;
+        float bv = s_val[0][mi];
+        int bi = s_idx[0][mi];
+#pragma unroll
+        for (int w = 1; w < 4; ++w) {
+            if (argmax_better(s_val[w][mi], s_idx[w][mi], bv, bi)) {
+                bv = s_val[w][mi];
+                bi = s_idx[w][mi];
+            }
+        }
+        if (m0 + mi < a.M) fin_m[0] = m0 + mi;
+        fin_key[0] = bi == INT_MAX ? 0ull : pack_argmax(bv, (uint32_t)bi);
+    }
+    tiled_argmax_finish(a, fin_m, fin_key, &s_last);
+}
+
+template <int RG, int KSTEPS, bool ROWMAJOR, typename BaseT, typename PriorT, bool VEC, bool HAS_PRIOR>
+hipError_t launch_rows_inst(const ArgmaxKArgs& ka, hipStream_t s) {
+    const int ntiles = (ka.V + 15) / 16;
+    const int groups = (ka.M + 16 * RG - 1) / (16 * RG);
+    const int cus = device_cu_count();
+    const int gx = std::max(1, std::min((ntiles + 3) / 4, (cus + groups - 1) / groups));
+    hipLaunchKernelGGL((fused_argmax_rows_kernel<RG, KSTEPS, ROWMAJOR, BaseT, PriorT, VEC, HAS_PRIOR>),
+                       dim3(gx, groups, 1), dim3(rows::kThreads), 0, s, ka);
+    return hipGetLastError();
+}
+
+// Whether launch_rows_* takes a prior of this kind beside base logits of BaseT:
+// none, the base's own dtype, or fp32.
+inline bool rows_prior_ok(int base_dtype, int prior_kind) {
+    return prior_kind == 0 || prior_kind == 1 || prior_kind == (base_dtype == 1 ? 2 : base_dtype == 2 ? 3 : 1);
+}
+
+// Dispatch over row groups, K steps / B layout, prior and vector loads for one
+// base dtype (rows_rank_ok).  `vec`: every row of base (and the prior) allows
+// aligned loads of four elements, V is a multiple of 4 and base spans under 4 GiB.
+template <typename BaseT>
+hipError_t launch_rows_for_base(const ArgmaxKArgs& ka, bool packed, int prior_kind, bool vec, hipStream_t s) {
+    using True = std::true_type;
+    using False = std::false_type;
+    auto by_shape = [&](auto prior_tag, auto has_tag, auto vec_tag) -> hipError_t {
+        using PriorT = decltype(prior_tag);
+        constexpr bool HP = decltype(has_tag)::value;
+        constexpr bool VEC = decltype(vec_tag)::value;
+        auto by_rows = [&](auto ks_tag, auto rm_tag) -> hipError_t {
+            constexpr int KS = decltype(ks_tag)::value;
+            constexpr bool RM = decltype(rm_tag)::value;
+            if (ka.M <= 32) return launch_rows_inst<2, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+            return launch_rows_inst<rows::max_groups<KS, BaseT, VEC>(), KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+        };
+        auto by_layout = [&](auto ks_tag) -> hipError_t {
+            return packed ? by_rows(ks_tag, False{}) : by_rows(ks_tag, True{});
+        };
+        if (ka.r == 512) return by_layout(std::integral_constant<int, 16>{});
+        if (ka.r == 256) return by_layout(std::integral_constant<int, 8>{});
+        return by_layout(std::integral_constant<int, 4>{});
+    };
+    auto by_vec = [&](auto prior_tag, auto has_tag) -> hipError_t {
+        return vec ? by_shape(prior_tag, has_tag, True{}) : by_shape(prior_tag, has_tag, False{});
+    };
+    if (prior_kind == 0) return by_vec(BaseT{}, False{});
+    if (prior_kind == 1) return by_vec(float{}, True{});
+    return by_vec(BaseT{}, True{});
+}
+
+hipError_t launch_rows_f32(const ArgmaxKArgs& ka, bool packed, int prior_kind, bool vec, hipStream_t s);
+hipError_t launch_rows_bf16(const ArgmaxKArgs& ka, bool packed, int prior_kind, bool vec, hipStream_t s);
+hipError_t launch_rows_f16(const ArgmaxKArgs& ka, bool packed, int prior_kind, bool vec, hipStream_t s);
+
+}  // namespace dels

@@ -100,8 +100,8 @@ struct TiledKArgs {
 // replaces a second kernel that reduced per-chunk keys: its launch cost more
 // than the atomics, which are spread over the workgroups' ends.)  `flag` may
 // alias the stage buffers: the first barrier ends every wave's use of them.
-template <int NB>
-__device__ __forceinline__ void tiled_argmax_finish(const TiledKArgs& a, const int (&m)[NB],
+template <int NB, typename Args>
+__device__ __forceinline__ void tiled_argmax_finish(const Args& a, const int (&m)[NB],
                                                     const unsigned long long (&key)[NB], int* flag) {
     __syncthreads();
     unsigned long long seen = 0;

@@ -121,7 +121,8 @@ def test_sample_rows_skipped_candidates_change_nothing(pkg, dev, dtype, V, pad):
     x[4, torch.rand(V, generator=g) < 0.9] = float("-inf")
     x[5, V - 1] = x[5, V // 3] = float("inf")     # the lowest of two infinities
     x[6, V - 1] = x[6, V // 2] = float("nan")     # the first NaN
-    x[7] *= 40.0                                  # float16: quotients near its largest value
+    x[7] *= 40.0
+    x[8] = (x[8].float() * 11000.0).clamp(-45500.0, 45500.0).to(dtype)   # float16: quotients up to its largest
     full = full.to(dev)
     ids, score = pkg.sample_rows(full[:, :V], T, seed)
     torch.cuda.synchronize()
