@@ -24,7 +24,7 @@ SOURCES = ["capi.hip", "skinny_gemm.hip", "fused_argmax.hip", "fused_argmax_f32.
            "fused_argmax_rows_f16.hip", "fused_argmax_tiled_f32.hip", "fused_argmax_tiled_bf16.hip",
            "fused_argmax_tiled_f16.hip", "lowrank_decode_f32.hip", "lowrank_decode_bf16.hip",
            "lowrank_decode_f16.hip", "pack.hip", "sample.hip", "domino_argmax.hip", "lm_head.hip",
-           "rollout_resident.hip"]
+           "rollout_resident.hip", "markov_resident.hip", "rollout_ordered.hip"]
 
 # -packed-fp32-ops: never emit v_pk_{add,mul,fma}_f32 (kept off on this target).
 HIP_FLAGS = [

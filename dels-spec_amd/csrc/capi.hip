@@ -442,6 +442,24 @@ static ArgmaxArgs gather_args(const int64_t* tokens, int64_t tok_stride, const v
 static int enqueue_markov(const dels_markov_rollout* p, hipStream_t s) {
     const size_t esz = dtype_size(p->base_dtype);
     const int64_t ldbase = p->ld_base ? p->ld_base : p->steps * p->V;
+    const bool packed = p->lm_layout == DELS_LAYOUT_MFMA16;
+    if (rollout_resident_enabled() &&
+        markov_resident_eligible(p->batch, p->r, p->V, p->steps, packed, p->ws_bytes)) {
+        // every step in one launch with B held on chip (markov_resident.hip)
+        MarkovRolloutArgs a{};
+        a.embedding = static_cast<const uint16_t*>(p->embedding);
+        a.ld_embedding = p->ld_embedding;
+        a.table_rows = p->table_rows;
+        a.B = static_cast<const uint16_t*>(p->lm_w);
+        a.base = p->base; a.ld_base = ldbase; a.base_dtype = p->base_dtype;
+        a.prior = p->prior; a.prior_dtype = p->prior_dtype;
+        a.alpha = p->alpha; a.beta = p->beta;
+        a.prev_ids = p->prev_ids; a.ld_prev = 1;
+        a.M = (int)p->batch; a.r = (int)p->r; a.V = (int)p->V; a.steps = (int)p->steps;
+        a.out_ids = p->out_ids; a.out_scores = p->out_scores; a.ld_out = p->steps;
+        hipError_t e = launch_markov_resident(a, p->ws, s);
+        return e == hipSuccess ? DELS_OK : hip_fail(e, "resident Markov rollout launch");
+    }
     for (int64_t step = 0; step < p->steps; ++step) {
         // token_s: the previous token for the first step, then the step before's pick
         const int64_t* tok = step == 0 ? p->prev_ids : p->out_ids + (step - 1);
@@ -1138,8 +1156,9 @@ int dels_gather_argmax(const int64_t* tokens, int64_t tok_stride, const void* E,
 
 size_t dels_markov_rollout_ws_bytes(int64_t batch, int64_t r, int64_t V) {
     if (!rows_ok(batch) || !rows_ok(r) || !vocab_ok(V)) return 0;
-    return kDataOff + align256(argmax_data_bytes(std::max<int64_t>(batch, 1), std::max<int64_t>(r, 1),
-                                                 std::max<int64_t>(V, 1)));
+    return kDataOff + std::max(align256(argmax_data_bytes(std::max<int64_t>(batch, 1), std::max<int64_t>(r, 1),
+                                                          std::max<int64_t>(V, 1))),
+                               kMarkovSlotBytes);
 }
 
 int dels_markov_rollout_enqueue(const dels_markov_rollout* p, void* stream) {

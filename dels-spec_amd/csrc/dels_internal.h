@@ -209,6 +209,33 @@ int resident_spin_limit();
 int set_resident_spin_limit(int limit);   // returns the previous limit
 int set_rollout_resident(int enable);   // returns the previous setting (1 = used where eligible)
 bool rollout_resident_enabled();
+// The Markov rollout with B resident on chip (markov_resident.hip: r = 128 or
+// 256, batch <= 32), followed on the stream by the ordered rollout, which does
+// the work when the resident launch could not get every CU and returns at once
+// otherwise.  The launchers fill the fields below the outputs.
+struct MarkovRolloutArgs {
+    const uint16_t* embedding; int64_t ld_embedding; int64_t table_rows;
+    const uint16_t* B;                                   // [V, r] MFMA-16 blocks
+    const void* base; int64_t ld_base; int base_dtype;   // row m, step s at base + m * ld_base + s * V (elements)
+    const void* prior; int prior_dtype;
+    const float* alpha; const float* beta;               // [steps]
+    const int64_t* prev_ids; int64_t ld_prev;
+    int M, r, V, steps;
+    int64_t* out_ids; float* out_scores; int64_t ld_out; // row m, step s at [m * ld_out + s]
+    int ntiles, mp_shift;
+    unsigned int* counters;                              // control area
+    unsigned long long* keys;                            // control area: argmax keys
+    unsigned long long* words;                           // arrival words, a line per workgroup
+    unsigned long long* slots;
+    int spin_limit, arrival_limit;
+};
+// Its slot words [parity][group of 16 rows][workgroup][16] lie in the data region
+// (a launch clears them before use), its arrival words where the other resident
+// rollout keeps its state words.
+constexpr size_t kMarkovSlotBytes = align256((size_t)4 * 16 * kResidentMaxWGs * 8);
+bool markov_resident_eligible(int64_t batch, int64_t r, int64_t V, int64_t steps, bool packed, size_t ws_bytes);
+hipError_t launch_markov_resident(MarkovRolloutArgs a, void* ws, hipStream_t s);
+hipError_t launch_markov_ordered(const MarkovRolloutArgs& a, hipStream_t s);
 // The fp8 decode step (A e4m3 K32, B e4m3 K128): as above with r in {128, 256, 512}.
 bool decode8_eligible(int64_t M, int64_t d, int64_t r);
 // A rollout step with the local head's GRU fused into the decode launch:

@@ -28,8 +28,8 @@
  *    the one-launch rollout advance once per launch (a launch generation) -- so no call needs a
  *    memset; then 544 KiB that only the fused decode step writes (its rank
  *    hand-off words, each tagged with a launch generation) and 144 KiB that
- *    only the one-launch rollout writes (its state and rank words, tagged with
- *    the launch generation and the step, and its argmax slot words, which each
+ *    only the one-launch rollouts write (state, rank and arrival words, tagged with
+ *    the launch generation and the step, and argmax slot words, which each
  *    launch clears before use); then data regions that may hold
  *    anything between calls.  One workspace may therefore serve
  *    every entry point and shape in turn; calls that share it must not
@@ -221,14 +221,16 @@ int dels_debug_set_decode_spin_limit(int limit);
  * (weights in the MFMA-16 layout, r = 256, batch <= 16, G <= 1024 a multiple of
  * twice the CU count, the vocabulary's share fitting a CU), dels_rollout_enqueue
  * and dels_graph_create run every step of the rollout in one launch that keeps
- * the low-rank head resident on chip; enable = 0 selects the per-step launches
- * instead (for later calls), 1 restores the default.  Returns the previous
+ * the low-rank head resident on chip, and so do the Markov rollout's entry points
+ * where theirs does; enable = 0 selects the per-step launches instead (for
+ * later calls), 1 restores the default.  Returns the previous
  * setting.  Not thread-safe.
  */
 int dels_debug_set_rollout_resident(int enable);
 /* Test hook: the waits of that one-launch rollout re-read each other's results
  * at most `limit` times (default 65536) before the launch gives up; a launch
- * that gives up writes -1 ids for the steps it could not finish, and the next
+ * that gives up writes -1 ids for the steps it could not finish (the Markov
+ * rollout: leaves the whole rollout to the launch that follows it), and the next
  * launch starts clean.  Returns the previous limit.  Not thread-safe. */
 int dels_debug_set_resident_spin_limit(int limit);
 
@@ -499,7 +501,13 @@ int dels_gather_argmax(const int64_t* tokens, int64_t tok_stride, const void* E,
  * The Markov rollout of MarkovDeLSGraphRunner._forward_impl
  * (code/kernel/markov_dels.py:261-278): token_0 = prev_ids; for each step s,
  * out_ids[:, s] = dels_gather_argmax(token_s) against base[:, s, :] with
- * alpha[s]/beta[s], and token_{s+1} = out_ids[:, s].  One launch per step.
+ * alpha[s]/beta[s], and token_{s+1} = out_ids[:, s].  With lm_w in the MFMA-16
+ * layout, r = 128 or 256, batch <= 32 and a vocabulary share that fits a CU, one
+ * launch that holds lm_w on chip does every step; it is followed by one that does
+ * the rollout in its place when it could not get every CU of the GPU (other
+ * streams or processes at work on it) and otherwise returns at once.  One launch
+ * per step for other shapes, and with a workspace below
+ * dels_markov_rollout_ws_bytes() that still holds the control area and words.
  */
 typedef struct dels_markov_rollout {
     const void* embedding;  /* [table_rows, r] bf16 row-major */
