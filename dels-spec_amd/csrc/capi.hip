@@ -262,7 +262,7 @@ static int enqueue_rollout(const dels_rollout* p, hipStream_t s) {
     uint16_t* h_next = static_cast<uint16_t*>(p->h_b);
     const size_t esz = dtype_size(p->base_dtype);
     const bool packed = p->weights_layout == DELS_LAYOUT_MFMA16;
-    if (rollout_resident_enabled() && rollout_resident_eligible(B, G, r, V, p->steps, packed)) {
+    if (rollout_resident_enabled() && rollout_resident_eligible(B, G, r, V, p->steps, packed, p->ws_bytes)) {
         // every step in one launch with B held on chip (rollout_resident.hip)
         ResidentRolloutArgs ra{};
         ra.w_hh = g.w_hh; ra.b_hh = g.b_hh;
@@ -277,6 +277,7 @@ static int enqueue_rollout(const dels_rollout* p, hipStream_t s) {
         ra.alpha = p->alpha; ra.beta = p->beta;
         ra.batch = B; ra.G = G; ra.V = V; ra.steps = p->steps;
         ra.out_ids = p->out_ids; ra.out_scores = p->out_scores; ra.ld_out = ldo;
+        ra.h_a = h_cur; ra.h_b = h_next; ra.rank = static_cast<uint16_t*>(p->rank);
         hipError_t e = launch_rollout_resident(ra, ws, s);
         return e == hipSuccess ? DELS_OK : hip_fail(e, "resident rollout launch");
     }
@@ -1113,8 +1114,10 @@ int dels_gru_step(const void* gi_table, int64_t ld_gi, int64_t table_rows, const
 
 size_t dels_rollout_ws_bytes(int64_t batch, int64_t G, int64_t r, int64_t V) {
     if (!rows_ok(batch) || !rows_ok(G) || !rows_ok(r) || !vocab_ok(V)) return 0;
-    return rollout_layout(std::max<int64_t>(batch, 1), std::max<int64_t>(G, 1), std::max<int64_t>(r, 1),
-                          std::max<int64_t>(V, 1)).total;
+    const size_t total = rollout_layout(std::max<int64_t>(batch, 1), std::max<int64_t>(G, 1), std::max<int64_t>(r, 1),
+                                        std::max<int64_t>(V, 1)).total;
+    // room for the one-launch rollout of two row groups where the batch may take it
+    return batch > 16 && batch <= 32 && r == kResidentRank ? std::max(total, kDataOff + kResident2Bytes) : total;
 }
 
 int dels_rollout_enqueue(const dels_rollout* p, void* stream) {

@@ -202,9 +202,16 @@ struct ResidentRolloutArgs {
     const float* alpha; const float* beta;
     int64_t batch, G, V, steps;
     int64_t* out_ids; float* out_scores; int64_t ld_out;   // row m, step s at [m * ld_out + s]
+    uint16_t* h_a; uint16_t* h_b; uint16_t* rank;          // the caller's state and rank buffers (ordered rollout)
 };
-bool rollout_resident_eligible(int64_t batch, int64_t G, int64_t r, int64_t V, int64_t steps, bool packed);
+// 17 to 32 rows run as two groups of 16, whose words lie in the data region (a
+// launch clears them before use), and are followed by the ordered rollout, which
+// does the work when the resident launch could not get every CU.
+constexpr size_t kResident2Bytes = 2 * kResidentWordBytes;
+bool rollout_resident_eligible(int64_t batch, int64_t G, int64_t r, int64_t V, int64_t steps, bool packed,
+                               size_t ws_bytes);
 hipError_t launch_rollout_resident(const ResidentRolloutArgs& a, void* ws, hipStream_t s);
+hipError_t launch_rollout_ordered(const ResidentRolloutArgs& a, void* ws, hipStream_t s);
 int resident_spin_limit();
 int set_resident_spin_limit(int limit);   // returns the previous limit
 int set_rollout_resident(int enable);   // returns the previous setting (1 = used where eligible)

@@ -342,4 +342,23 @@ hipError_t launch_markov_ordered(const MarkovRolloutArgs& r, hipStream_t s) {
     return launch_ordered_base<false, 4>(a, r.prior, r.prior_dtype, r.base_dtype, s);
 }
 
+hipError_t launch_rollout_ordered(const ResidentRolloutArgs& r, void* ws, hipStream_t s) {
+    char* w = static_cast<char*>(ws);
+    OrderedArgs a{};
+    a.w_hh = r.w_hh; a.b_hh = r.b_hh;
+    a.A = r.A; a.rank_b = r.rank_b; a.act = r.act;
+    a.gi_table = r.gi_table; a.ld_gi = r.ld_gi; a.table_rows = r.table_rows; a.G = (int)r.G;
+    a.h[0] = r.h_a; a.h[1] = r.h_b; a.rank = r.rank;
+    a.B = r.B;
+    a.base = r.base; a.ld_base = r.ld_base;
+    a.prior = r.prior;
+    a.alpha = r.alpha; a.beta = r.beta;
+    a.first_ids = r.prefix; a.ld_first = r.ld_prefix;
+    a.M = (int)r.batch; a.V = (int)r.V; a.steps = (int)r.steps; a.ntiles = (int)((r.V + 15) / 16);
+    a.out_ids = r.out_ids; a.out_scores = r.out_scores; a.ld_out = r.ld_out;
+    a.counters = reinterpret_cast<unsigned int*>(w + kCountersOff);
+    a.keys = reinterpret_cast<unsigned long long*>(w + kKeysOff);
+    return launch_ordered_base<true, kResidentRank / 32>(a, r.prior, r.prior_dtype, r.base_dtype, s);
+}
+
 }  // namespace dels

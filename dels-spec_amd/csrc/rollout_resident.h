@@ -58,12 +58,13 @@ struct RrWords {
     int row;      // log2 of the words per row
     int mp;       // log2 of the rows rounded up
     int M;        // rows present
+    int split = INT_MAX, M2 = 0;   // from word `split` on: a second group, of M2 rows
     __device__ __forceinline__ uint32_t addr(int j) const {
         j = j < n ? j : n - 1;   // past the end: the last word again (loaded, never examined)
         return ((uint32_t)(j >> blk) << stride) + (uint32_t)(j & ((1 << blk) - 1));
     }
     __device__ __forceinline__ int row_of(int j) const { return (j >> row) & ((1 << mp) - 1); }
-    __device__ __forceinline__ bool live(int j) const { return j < n && row_of(j) < M; }
+    __device__ __forceinline__ bool live(int j) const { return j < n && row_of(j) < (j < split ? M : M2); }
 };
 
 // Load the words j = tid + kRrThreads * i, i < NPT -- every load issued before

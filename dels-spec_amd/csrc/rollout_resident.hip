@@ -45,6 +45,11 @@
 // -1, and the launch still ends (every workgroup reaches the end, the last
 // one resets the error word and advances the generation).  The workgroups
 // must be resident at once (one per CU) for the waits to succeed.
+//
+// Up to 16 rows run as one group.  17 to 32 run as two (see the kernel); a launch
+// that cannot finish them leaves the rollout to the ordered one behind it.  14
+// steps of 24 rows at V = 151936, G = 1024, with the copies of a runner's call:
+// 577.9 us as per-step launches (argmax 17 us, GRU 8.6, rank 7.7 a step), 307.9 here.
 #include <algorithm>
 #include <climits>
 
@@ -78,23 +83,32 @@ struct RrArgs {
     unsigned int* counters;                         // control area
     unsigned long long* h_words;                    // per workgroup: rows x upw/2 words, on lines of its own
     unsigned long long* rank_words;                 // per rank workgroup: rows x 8 words
-    unsigned long long* slots;                      // [2][nwg][16]: parity, workgroup (a line each), row
+    unsigned long long* slots;                      // [2][RG][nwg][16]: parity, group, workgroup (a line each), row
+    unsigned long long* arrivals;                   // two groups: a word per workgroup, on lines of their own
     int spin_limit;
 };
 
-template <typename BaseT, typename PriorT>
+// RG: groups of 16 rows.  With two, the even workgroups advance the GRU (and the
+// rank) of rows 0..15 and the odd ones that of rows 16..: each group's state is
+// exchanged among half the workgroups, which own twice the units, so that no
+// workgroup reads more state words than with 16 rows; every workgroup contracts
+// its tiles of B with both groups' ranks.  A group's rows are numbered from its
+// first: M rows of the group from row m0 of the batch.
+template <int RG, typename BaseT, typename PriorT>
 __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) {
 #pragma clang fp contract(off)
+    constexpr int kUnitTiles = RG;                  // operand tiles of W_hh rows: RG * 4 units x 3 gates
+    constexpr int kGhPitch = 16 * kUnitTiles;
     __shared__ __attribute__((aligned(16))) uint16_t s_h[16 * kRrHPitch];        // the state, rows >= M zero
     __shared__ __attribute__((aligned(16))) char s_whh[(kResidentMaxG / 32) * 1024];   // W_hh rows of the units
     __shared__ __attribute__((aligned(16))) char s_union[kRrUnionBytes];       // A rows (rank WGs) or B tiles
-    __shared__ __attribute__((aligned(16))) uint16_t s_rank[16 * kRrRPitch];
-    __shared__ __attribute__((aligned(16))) float s_red[kRrWaves * 256];
+    __shared__ __attribute__((aligned(16))) uint16_t s_rank[RG * 16 * kRrRPitch];
+    __shared__ __attribute__((aligned(16))) float s_red[RG * kRrWaves * 256];
     __shared__ float s_prior[(kRrWaves * kRrRegTiles + kResidentLdsTiles) * 16];
-    __shared__ unsigned long long s_key[kRrWaves][16];    // each wave's best key of each row
-    __shared__ float s_gh[16 * 16];
+    __shared__ unsigned long long s_key[kRrWaves][RG * 16];    // each wave's best key of each row
+    __shared__ float s_gh[16 * kGhPitch];
     __shared__ float s_ab[2][kResidentMaxSteps];          // alpha, beta of each step
-    __shared__ float s_bias[32];                          // b_hh of the operand rows, rank bias of the tile
+    __shared__ float s_bias[16 * kUnitTiles + 16];                        // b_hh of the operand rows, rank bias of the tile
     __shared__ unsigned long long s_rowmax[16];           // the step's maximum slot word of each row
     __shared__ int64_t s_ids[16];
     __shared__ int s_flag;
@@ -103,22 +117,25 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int col = lane & 15, kg = lane >> 4;
     const int w = blockIdx.x, nwg = gridDim.x;
-    const int G = a.G, KB = G / 32, M = a.M, V = a.V;
+    const int grp = RG == 2 ? (w & 1) : 0, wg = RG == 2 ? w >> 1 : w, ng = nwg / RG;   // group, place in it, its size
+    const int m0 = 16 * grp;
+    const int G = a.G, KB = G / 32, V = a.V;
+    const int M = RG == 2 ? (grp ? a.M - 16 : 16) : a.M;
     const uint32_t gen = __hip_atomic_load(a.counters + kDecodeGenWord, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const BaseT* base = static_cast<const BaseT*>(a.base);
     const PriorT* prior = static_cast<const PriorT*>(a.prior);
-    const bool rank_wg = w < kRrRankWGs;
+    const bool rank_wg = wg < kRrRankWGs;
 
     // ---- this workgroup's vocabulary tiles [T0, T1): 32 for a rank workgroup, the
     // rest shared evenly by the others (the plan checks they fit)
     int T0, T1;
     {
-        const int first = min(a.ntiles, kRrRankWGs * kRrWaves * kRrRegTiles);
+        const int first = min(a.ntiles, RG * kRrRankWGs * kRrWaves * kRrRegTiles);
         if (rank_wg) {
             T0 = min(a.ntiles, w * kRrWaves * kRrRegTiles);
             T1 = min(a.ntiles, T0 + kRrWaves * kRrRegTiles);
         } else {
-            const int rest = a.ntiles - first, j = w - kRrRankWGs, n = nwg - kRrRankWGs;
+            const int rest = a.ntiles - first, j = w - RG * kRrRankWGs, n = nwg - RG * kRrRankWGs;
             T0 = first + (int)(((int64_t)j * rest) / n);
             T1 = first + (int)(((int64_t)(j + 1) * rest) / n);
         }
@@ -128,25 +145,30 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     const int nlds = max(0, ntl - kRrWaves * kRrRegTiles);
     const bool has_lds_tile = wave < nlds;
 
-    const int u0 = w * a.upw;   // this workgroup's first GRU unit
+    const int u0 = wg * a.upw;   // this workgroup's first GRU unit
+    const int upt = RG == 2 ? min(a.upw, 4) : a.upw;   // units per operand tile
     for (int i = threadIdx.x; i < 16 * kRrHPitch / 2; i += kRrThreads) reinterpret_cast<uint32_t*>(s_h)[i] = 0u;
-    for (int i = threadIdx.x; i < 16 * kRrRPitch / 2; i += kRrThreads) reinterpret_cast<uint32_t*>(s_rank)[i] = 0u;
+    for (int i = threadIdx.x; i < RG * 16 * kRrRPitch / 2; i += kRrThreads) reinterpret_cast<uint32_t*>(s_rank)[i] = 0u;
     for (int i = threadIdx.x; i < a.steps; i += kRrThreads) {
         s_ab[0][i] = a.alpha[i];
         s_ab[1][i] = a.beta[i];
     }
     if (threadIdx.x < 16) {
         const int j = threadIdx.x;
-        float bh = 0.f, br = 0.f;
-        if (a.b_hh && j < 3 * a.upw) {
-            const int g = j / a.upw, u = u0 + (j - g * a.upw);
-            bh = bf16_bits_to_f32(a.b_hh[g * G + u]);
+        float br = 0.f;
+#pragma unroll
+        for (int t = 0; t < kUnitTiles; ++t) {
+            float bh = 0.f;
+            if (a.b_hh && j < 3 * upt && (RG == 1 || t * upt < a.upw)) {
+                const int g = j / upt, u = u0 + t * upt + (j - g * upt);
+                bh = bf16_bits_to_f32(a.b_hh[g * G + u]);
+            }
+            s_bias[16 * t + j] = bh;
         }
-        if (rank_wg && a.rank_b) br = bf16_bits_to_f32(a.rank_b[w * 16 + j]);
-        s_bias[j] = bh;
-        s_bias[16 + j] = br;
+        if (rank_wg && a.rank_b) br = bf16_bits_to_f32(a.rank_b[wg * 16 + j]);
+        s_bias[16 * kUnitTiles + j] = br;
         s_rowmax[j] = 0ull;
-    } else if (threadIdx.x < 48) {
+    } else if (RG == 1 && threadIdx.x < 48) {
         // this workgroup's slots of both parity sets back to zero; waiting for the
         // old values means the exchanges are done before the barrier below, so
         // before the prefix state words that every reader waits for
@@ -162,33 +184,73 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     // and rank workgroup), the argmax slots (one word per row and workgroup, a
     // line per workgroup)
     const int mp = a.mp_shift;
-    const RrWords h_pl{nwg << (mp + a.np_shift), mp + a.np_shift, max(4, mp + a.np_shift), a.np_shift, mp, M};
+    const RrWords h_pl{ng << (mp + a.np_shift), mp + a.np_shift, max(4, mp + a.np_shift), a.np_shift, mp, M};
     const RrWords r_pl{kRrRankWGs << (mp + 3), mp + 3, mp + 3, 3, mp, M};
     const RrWords s_pl{nwg << mp, mp, 4, 0, mp, M};
+    // each group's words in a region of their own (one group: the region)
+    unsigned long long* const h_words = a.h_words + (RG == 2 ? grp * (int)(kResidentHWordBytes / 8) : 0);
+    constexpr int kRankGroup = (int)(kResidentRankWordBytes / 8);
+    unsigned long long* const rank_words = a.rank_words + (RG == 2 ? grp * kRankGroup : 0);
+    const uint32_t atag = rr_tag(gen, 255);
+    bool ok = true;
+    if constexpr (RG == 2) {
+        // The words lie in the data region, where anything may have been left: each
+        // workgroup clears the words it will write and only then publishes an
+        // arrival word (in the region of tagged words); everyone waits for all
+        // arrivals (below) before it reads any other word.  The wait is short and
+        // also tells whether the whole grid is resident.
+        const int nh = 1 << h_pl.stride;                  // state words of this workgroup
+        const int nr = rank_wg ? 1 << r_pl.stride : 0;
+        for (int i = threadIdx.x; i < nh + nr + 64; i += kRrThreads) {
+            unsigned long long* p = i < nh ? h_words + ((int64_t)wg << h_pl.stride) + i
+                                    : i < nh + nr ? rank_words + ((int64_t)wg << r_pl.stride) + (i - nh)
+                                    : a.slots + ((i - nh - nr) >> 4) * kRrSlotSet + w * 16 + ((i - nh - nr) & 15);
+            const unsigned long long old = __hip_atomic_exchange(p, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("" ::"v"(old));
+        }
+        __syncthreads();
+        if (threadIdx.x == 0)
+            __hip_atomic_store(a.arrivals + w * 16, (unsigned long long)atag << 32, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
 
     // ---- pieces of a step ----------------------------------------------------------
     // gh of the workgroup's units from the state in s_h (zero previous state:
     // no product) into s_gh[m * 16 + j], bf16-rounded after the bias.
     auto compute_gh = [&](bool zero_state) __attribute__((always_inline)) {
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        f32x4 acc[kUnitTiles];
+#pragma unroll
+        for (int t = 0; t < kUnitTiles; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
         if (!zero_state) {
             for (int kb = wave; kb < KB; kb += kRrWaves) {
                 const bf16x8 hv = *reinterpret_cast<const bf16x8*>(&s_h[col * kRrHPitch + kb * 32 + kg * 8]);
                 const bf16x8 wv = *reinterpret_cast<const bf16x8*>(s_whh + kb * 1024 + lane * 16);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hv, wv, acc, 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(hv, wv, acc[0], 0, 0, 0);
+                if constexpr (RG == 2) {
+                    // the second tile's rows do not fit the LDS beside the rest: from the L2 every step
+                    const int g = col / upt, row = g * G + u0 + upt + (col - g * upt);
+                    const bool live = col < 3 * upt && upt < a.upw;
+                    const u32x4 w1 = *reinterpret_cast<const u32x4*>(
+                        a.w_hh + ((int64_t)((live ? row : 0) >> 4) * KB + kb) * 512 + ((live ? row & 15 : 0) + 16 * kg) * 8);
+                    acc[kUnitTiles - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        hv, masked_bf16x8(w1, live ? ~0u : 0u), acc[kUnitTiles - 1], 0, 0, 0);
+                }
             }
         }
-        *reinterpret_cast<f32x4*>(&s_red[wave * 256 + lane * 4]) = acc;
+#pragma unroll
+        for (int t = 0; t < kUnitTiles; ++t)
+            *reinterpret_cast<f32x4*>(&s_red[t * kRrWaves * 256 + wave * 256 + lane * 4]) = acc[t];
         __syncthreads();
-        if (threadIdx.x < 256) {
+        if (RG == 2 || threadIdx.x < 256) {
             // element (row m, operand row j): lane (m/4)*16 + j, entry m%4
-            const int m = threadIdx.x >> 4, j = threadIdx.x & 15;
-            const int e = (((m >> 2) * 16 + j) << 2) + (m & 3);
+            const int t = RG == 2 ? (int)threadIdx.x >> 8 : 0;
+            const int m = (threadIdx.x & 255) >> 4, j = threadIdx.x & 15;
+            const int e = t * kRrWaves * 256 + ((((m >> 2) * 16 + j) << 2) + (m & 3));
             float v = s_red[e];
 #pragma unroll
             for (int ww = 1; ww < kRrWaves; ++ww) v = v + s_red[ww * 256 + e];
-            if (a.b_hh) v = v + s_bias[j];
-            s_gh[m * 16 + j] = round_bf16(v);
+            if (a.b_hh) v = v + s_bias[16 * t + j];
+            s_gh[m * kGhPitch + 16 * t + j] = round_bf16(v);
         }
         __syncthreads();
     };
@@ -210,13 +272,14 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 const int i = 2 * p + h, u = u0 + i;
+                const int gi0 = RG == 2 && i >= upt ? m * kGhPitch + 16 + i - upt : m * kGhPitch + i;   // gate r of unit i
                 const float hv = bf16_bits_to_f32(s_h[m * kRrHPitch + u]);
                 const float v = gru_unit(bf16_bits_to_f32(gv[0][h]), bf16_bits_to_f32(gv[1][h]),
-                                         bf16_bits_to_f32(gv[2][h]), s_gh[m * 16 + i],
-                                         s_gh[m * 16 + a.upw + i], s_gh[m * 16 + 2 * a.upw + i], hv);
+                                         bf16_bits_to_f32(gv[2][h]), s_gh[gi0], s_gh[gi0 + upt],
+                                         s_gh[gi0 + 2 * upt], hv);
                 pair |= (uint32_t)f32_to_bf16_bits(v) << (16 * h);
             }
-            __hip_atomic_store(a.h_words + h_pl.addr((m << a.np_shift) + p + (w << h_pl.blk)),
+            __hip_atomic_store(h_words + h_pl.addr((m << a.np_shift) + p + (wg << h_pl.blk)),
                                ((unsigned long long)tag << 32) | pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
@@ -227,9 +290,9 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
             return reinterpret_cast<uint32_t*>(&s_h[m * kRrHPitch + wp * a.upw + 2 * p]);
         };
         // as few loads per thread as cover the words
-        if (h_pl.n <= 4 * kRrThreads) return rr_read_words<4>(a, a.h_words, h_pl, tag, map);
-        if (h_pl.n <= 8 * kRrThreads) return rr_read_words<8>(a, a.h_words, h_pl, tag, map);
-        return rr_read_words<16>(a, a.h_words, h_pl, tag, map);
+        if (h_pl.n <= 4 * kRrThreads) return rr_read_words<4>(a, h_words, h_pl, tag, map);
+        if (h_pl.n <= 8 * kRrThreads) return rr_read_words<8>(a, h_words, h_pl, tag, map);
+        return rr_read_words<16>(a, h_words, h_pl, tag, map);
     };
     // rank workgroup: its 16 columns of the rank from s_h, published as words
     auto rank_publish = [&](uint32_t tag) __attribute__((always_inline)) {
@@ -252,41 +315,49 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
                     float v = s_red[e];
 #pragma unroll
                     for (int ww = 1; ww < kRrWaves; ++ww) v = v + s_red[ww * 256 + e];
-                    if (a.rank_b) v = v + s_bias[16 + n];
+                    if (a.rank_b) v = v + s_bias[16 * kUnitTiles + n];
                     v = round_bf16(v);
                     if (a.act == 1) v = round_bf16(silu_f32(v));
                     pair |= (uint32_t)f32_to_bf16_bits(v) << (16 * h);
                 }
-                __hip_atomic_store(a.rank_words + r_pl.addr((w << r_pl.blk) + (m << 3) + p),
+                __hip_atomic_store(rank_words + r_pl.addr((wg << r_pl.blk) + (m << 3) + p),
                                    ((unsigned long long)tag << 32) | pair, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
         }
         __syncthreads();   // s_red is reused
     };
     auto read_rank = [&](uint32_t tag) __attribute__((always_inline)) -> bool {
+        if constexpr (RG == 2) {
+            // both groups' words in one gather: producer wr of group wr / kRrRankWGs
+            const RrWords pl{2 * kRrRankWGs << 7, 7, 7, 3, 4, 16, kRrRankWGs << 7, a.M - 16};
+            auto map = [&](int j) {
+                const int m = pl.row_of(j) + 16 * (j >> 11), wr = (j >> 7) & (kRrRankWGs - 1), p = j & 7;
+                return reinterpret_cast<uint32_t*>(&s_rank[m * kRrRPitch + wr * 16 + 2 * p]);
+            };
+            return rr_read_words<8>(a, a.rank_words, pl, tag, map);
+        }
         auto map = [&](int j) {
             const int m = r_pl.row_of(j), wr = j >> r_pl.blk, p = j & 7;
             return reinterpret_cast<uint32_t*>(&s_rank[m * kRrRPitch + wr * 16 + 2 * p]);
         };
-        if (r_pl.n <= 2 * kRrThreads) return rr_read_words<2>(a, a.rank_words, r_pl, tag, map);
-        return rr_read_words<4>(a, a.rank_words, r_pl, tag, map);
+        if (r_pl.n <= 2 * kRrThreads) return rr_read_words<2>(a, rank_words, r_pl, tag, map);
+        return rr_read_words<4>(a, rank_words, r_pl, tag, map);
     };
 
 
     // ---- prefix: h_0 = GRU(gi_table[prefix], 0) --------------------------------
-    bool ok = true;
     compute_gh(true);
-    gru_publish(a.prefix, a.ld_prefix, rr_tag(gen, 0));
+    gru_publish(a.prefix + m0 * a.ld_prefix, a.ld_prefix, rr_tag(gen, 0));
 
     // ---- resident operands, loaded while the prefix state travels (a read
     // waits for every load issued before it, so the state went out first):
     // the LDS operands, then this wave's register tiles of B
     if (rank_wg) {
-        // A rows 16 w .. 16 w + 15: the MFMA-16 blocks of that row block, in order
+        // A rows 16 wg .. 16 wg + 15: the MFMA-16 blocks of that row block, in order
         for (int i = threadIdx.x; i < KB * 64; i += kRrThreads) {
             const int kb = i >> 6, l = i & 63;
             *reinterpret_cast<u32x4*>(s_union + kb * 1024 + l * 16) =
-                *reinterpret_cast<const u32x4*>(a.A + ((int64_t)w * KB + kb) * 512 + l * 8);
+                *reinterpret_cast<const u32x4*>(a.A + ((int64_t)wg * KB + kb) * 512 + l * 8);
         }
     } else {
         for (int i = threadIdx.x; i < nlds * kRrKs * 64; i += kRrThreads) {
@@ -296,14 +367,14 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
                 *reinterpret_cast<const u32x4*>(a.B + ((int64_t)t * kRrKs + s) * 512 + l * 8);
         }
     }
-    // W_hh rows of units u0 .. u0 + upw - 1: operand row j = g * upw + i holds row
-    // g * G + u0 + i of W_hh (rows past 3 upw are zero)
+    // W_hh rows of the first operand tile, units u0 .. u0 + upt - 1: operand row
+    // j = g * upt + i holds row g * G + u0 + i of W_hh (rows past 3 upt are zero)
     for (int i = threadIdx.x; i < KB * 64; i += kRrThreads) {
         const int kb = i >> 6, l = i & 63;
         const int j = l & 15, oct = l >> 4;
         u32x4 v = {0u, 0u, 0u, 0u};
-        if (j < 3 * a.upw) {
-            const int g = j / a.upw, row = g * G + u0 + (j - g * a.upw);
+        if (j < 3 * upt) {
+            const int g = j / upt, row = g * G + u0 + (j - g * upt);
             v = *reinterpret_cast<const u32x4*>(a.w_hh + ((int64_t)(row >> 4) * KB + kb) * 512 + ((row & 15) + 16 * oct) * 8);
         }
         *reinterpret_cast<u32x4*>(s_whh + kb * 1024 + l * 16) = v;
@@ -330,7 +401,16 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
                                      keep);
     }
 
-    ok = read_state(rr_tag(gen, 0));
+    if constexpr (RG == 2) {
+        RrArgs first = a;
+        first.spin_limit = min(a.spin_limit, kRrArrivalLimit);
+        const RrWords pl{nwg, 0, 4, 0, 0, 1};
+        unsigned long long word[1];
+        const bool got = rr_gather<1>(first, a.arrivals, pl, (int)threadIdx.x, word,
+                                      [&](unsigned long long x) { return (uint32_t)(x >> 32) == atag; });
+        ok = !__syncthreads_or(!got);
+    }
+    if (ok) ok = read_state(rr_tag(gen, 0));
 
     int s = 0;
     for (; ok && s < a.steps; ++s) {
@@ -344,7 +424,7 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         // base values of this wave's tiles (issued before the rank wait): the
         // wave-uniform start of each tile's columns plus one per-lane offset per row
         uint32_t braw[kRrRegTiles + 1][4];
-        {
+        auto load_base = [&](int g) __attribute__((always_inline)) {
             const BaseT* bs = base + (int64_t)s * V;
 #pragma unroll
             for (int j = 0; j <= kRrRegTiles; ++j) {
@@ -353,11 +433,12 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
                 const int vc = min(tc * 16 + lcol, V - 1);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const int m = 4 * lkg + q;
-                    braw[j][q] = load_raw(bs + (int64_t)(m < M ? m : 0) * a.ld_base + vc);
+                    const int m = 16 * g + 4 * lkg + q;
+                    braw[j][q] = load_raw(bs + (int64_t)(m < a.M ? m : 0) * a.ld_base + vc);
                 }
             }
-        }
+        };
+        load_base(0);
         // keep these loads ahead of the rank wait (the compiler would otherwise
         // issue them after it, where their round trip adds to the step)
         asm volatile("" ::: "memory");
@@ -370,67 +451,72 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         const float al = s_ab[0][s], be = s_ab[1][s];
         const bool use_prior = !is_no_prior<PriorT>::value && be != 0.f;
         const bool lds_tile = !rank_wg && has_lds_tile;
-        f32x4 acc[kRrRegTiles + 1];
 #pragma unroll
-        for (int j = 0; j <= kRrRegTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // unconditional contractions (no branches between the MFMAs): a tile that
-        // is not this wave's holds zeros, or for the LDS slot of a wave without
-        // one any data, and is not combined
-        const int lslot = lds_tile ? wave : 0;
+        for (int g = 0; g < RG; ++g) {
+            if (g > 0) load_base(g);
+            f32x4 acc[kRrRegTiles + 1];
 #pragma unroll
-        for (int k = 0; k < kRrKs; ++k) {
-            const bf16x8 rk = *reinterpret_cast<const bf16x8*>(&s_rank[lcol * kRrRPitch + k * 32 + lkg * 8]);
-            const bf16x8 bv = *reinterpret_cast<const bf16x8*>(s_union + (lslot * kRrKs + k) * 1024 + lane * 16);
+            for (int j = 0; j <= kRrRegTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            // unconditional contractions (no branches between the MFMAs): a tile that
+            // is not this wave's holds zeros, or for the LDS slot of a wave without
+            // one any data, and is not combined
+            const int lslot = lds_tile ? wave : 0;
 #pragma unroll
-            for (int j = 0; j < kRrRegTiles; ++j)
-                acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bt[j][k], acc[j], 0, 0, 0);
-            acc[kRrRegTiles] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bv, acc[kRrRegTiles], 0, 0, 0);
-        }
-        float best[4];
-        int bidx[4];
+            for (int k = 0; k < kRrKs; ++k) {
+                const bf16x8 rk = *reinterpret_cast<const bf16x8*>(&s_rank[(16 * g + lcol) * kRrRPitch + k * 32 + lkg * 8]);
+                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(s_union + (lslot * kRrKs + k) * 1024 + lane * 16);
 #pragma unroll
-        for (int q = 0; q < 4; ++q) { best[q] = -__builtin_inff(); bidx[q] = INT_MAX; }
-        // a lane's column grows with its tile number, so a later tile takes the
-        // lead only on a larger score, or on an equal one while nothing has
-        // (the first -inf); written with bitwise tests, no branches
+                for (int j = 0; j < kRrRegTiles; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bt[j][k], acc[j], 0, 0, 0);
+                acc[kRrRegTiles] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bv, acc[kRrRegTiles], 0, 0, 0);
+            }
+            float best[4];
+            int bidx[4];
 #pragma unroll
-        for (int j = 0; j <= kRrRegTiles; ++j) {
-            const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
-            const bool live = j < kRrRegTiles ? ti < ntl : lds_tile;   // wave-uniform
-            const int tc = min(ti, max(ntl - 1, 0));
-            const int v = (T0 + tc) * 16 + lcol;
-            const bool livev = live & (v < V);
-            const float pv = s_prior[tc * 16 + lcol];
+            for (int q = 0; q < 4; ++q) { best[q] = -__builtin_inff(); bidx[q] = INT_MAX; }
+            // a lane's column grows with its tile number, so a later tile takes the
+            // lead only on a larger score, or on an equal one while nothing has
+            // (the first -inf); written with bitwise tests, no branches
+#pragma unroll
+            for (int j = 0; j <= kRrRegTiles; ++j) {
+                const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
+                const bool live = j < kRrRegTiles ? ti < ntl : lds_tile;   // wave-uniform
+                const int tc = min(ti, max(ntl - 1, 0));
+                const int v = (T0 + tc) * 16 + lcol;
+                const bool livev = live & (v < V);
+                const float pv = s_prior[tc * 16 + lcol];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    float sc = __builtin_fmaf(acc[j][q], al, widen_raw<BaseT>(braw[j][q]));
+                    if (use_prior) sc = __builtin_fmaf(-be, pv, sc);
+                    const bool take = livev & ((sc > best[q]) | ((sc == best[q]) & (bidx[q] == INT_MAX)));
+                    best[q] = take ? sc : best[q];
+                    bidx[q] = take ? v : bidx[q];
+                }
+            }
+            // over the 16 columns of each row as argmax keys (a lane without a
+            // candidate holds -inf at index INT_MAX, below every real one; DPP row
+            // shifts: lane 15 of a row ends with the row's best), then (below) the waves
+            unsigned long long key[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                float sc = __builtin_fmaf(acc[j][q], al, widen_raw<BaseT>(braw[j][q]));
-                if (use_prior) sc = __builtin_fmaf(-be, pv, sc);
-                const bool take = livev & ((sc > best[q]) | ((sc == best[q]) & (bidx[q] == INT_MAX)));
-                best[q] = take ? sc : best[q];
-                bidx[q] = take ? v : bidx[q];
+                key[q] = pack_argmax(best[q], (uint32_t)bidx[q]);
+                rr_row_max<1>(key[q]);
+                rr_row_max<2>(key[q]);
+                rr_row_max<4>(key[q]);
+                rr_row_max<8>(key[q]);
             }
-        }
-        // over the 16 columns of each row as argmax keys (a lane without a
-        // candidate holds -inf at index INT_MAX, below every real one; DPP row
-        // shifts: lane 15 of a row ends with the row's best), then (below) the waves
-        unsigned long long key[4];
+            if (col == 15) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            key[q] = pack_argmax(best[q], (uint32_t)bidx[q]);
-            rr_row_max<1>(key[q]);
-            rr_row_max<2>(key[q]);
-            rr_row_max<4>(key[q]);
-            rr_row_max<8>(key[q]);
-        }
-        if (col == 15) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) s_key[wave][4 * kg + q] = key[q];
+                for (int q = 0; q < 4; ++q) s_key[wave][16 * g + 4 * kg + q] = key[q];
+            }
         }
         __syncthreads();
         // the workgroup's best of each row into its slot word for the step
         const uint32_t low2 = 1u | ((((uint32_t)s >> 1) & 1u) << 1);
-        unsigned long long* slot_set = a.slots + (s & 1) * kRrSlotSet;
-        if ((int)threadIdx.x < M) {
+        unsigned long long* slot_set = a.slots + (s & 1) * RG * kRrSlotSet;
+        unsigned long long* const own_set = slot_set + (RG == 2 ? grp * kRrSlotSet : 0);
+        if ((int)threadIdx.x < a.M) {
             const int m = threadIdx.x;
             unsigned long long k = s_key[0][m];   // order(score) << 32 | ~index
 #pragma unroll
@@ -439,7 +525,8 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
             // 2^30 - 1, past every vocabulary, below every real candidate
             const unsigned long long word =
                 low2 | (k & 0xffffffff00000000ull) | ((unsigned long long)((uint32_t)k & 0x3fffffffu) << 2);
-            __hip_atomic_store(slot_set + w * 16 + m, word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(slot_set + (RG == 2 ? (m >> 4) * kRrSlotSet + w * 16 + (m & 15) : w * 16 + m), word,
+                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
 
         // next step's gh while the slot words travel (every workgroup: placed
@@ -448,11 +535,11 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         if (s + 1 < a.steps) compute_gh(false);
 
         // ---- the step's ids (every workgroup: its GRU units need them) ---------------
-        const bool need = s + 1 < a.steps || w == 0;
+        const bool need = s + 1 < a.steps || wg == 0;
         if (need) {
-            if (s_pl.n <= 2 * kRrThreads) ok = rr_slot_maxima<2>(a, slot_set, s_pl, low2, s_rowmax);
-            else if (s_pl.n <= 4 * kRrThreads) ok = rr_slot_maxima<4>(a, slot_set, s_pl, low2, s_rowmax);
-            else ok = rr_slot_maxima<8>(a, slot_set, s_pl, low2, s_rowmax);
+            if (s_pl.n <= 2 * kRrThreads) ok = rr_slot_maxima<2>(a, own_set, s_pl, low2, s_rowmax);
+            else if (s_pl.n <= 4 * kRrThreads) ok = rr_slot_maxima<4>(a, own_set, s_pl, low2, s_rowmax);
+            else ok = rr_slot_maxima<8>(a, own_set, s_pl, low2, s_rowmax);
             if (!ok) break;
             if (threadIdx.x < 16) {
                 const int m = threadIdx.x;
@@ -466,9 +553,9 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
                         id = idx;
                         val = f32_from_order_key((uint32_t)(key >> 32));
                     }
-                    if (w == 0) {
-                        a.out_ids[(int64_t)m * a.ld_out + s] = id;
-                        if (a.out_scores) a.out_scores[(int64_t)m * a.ld_out + s] = val;
+                    if (wg == 0) {
+                        a.out_ids[(int64_t)(m0 + m) * a.ld_out + s] = id;
+                        if (a.out_scores) a.out_scores[(int64_t)(m0 + m) * a.ld_out + s] = val;
                     }
                 }
                 s_ids[m] = id;
@@ -482,8 +569,8 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     }
     if (!ok) {
         if (threadIdx.x == 0) rr_fail(a);
-        // the ids this launch could not produce
-        if (w == 0) {
+        // the ids this launch could not produce (two groups: the ordered rollout produces them all)
+        if (RG == 1 && w == 0) {
             for (int i = threadIdx.x; i < M * a.steps; i += kRrThreads) {
                 const int m = i / a.steps, st = i - m * a.steps;
                 if (st >= s) {
@@ -497,6 +584,7 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     // ---- the last workgroup clears the control area and advances the generation
     __syncthreads();
     if (threadIdx.x == 0) {
+        __builtin_amdgcn_s_waitcnt(0);   // a failure is stored before this workgroup counts as done
         const unsigned prev = __hip_atomic_fetch_add(a.counters + kRrDoneCounter, 1u, __ATOMIC_RELAXED,
                                                      __HIP_MEMORY_SCOPE_AGENT);
         s_flag = prev == (unsigned)nwg - 1 ? 3 : 0;
@@ -504,22 +592,31 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     __syncthreads();
     if (s_flag != 3) return;
     if (threadIdx.x == 0) {
-        __hip_atomic_store(a.counters + kRrErrorWord, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const unsigned failed = __hip_atomic_exchange(a.counters + kRrErrorWord, 0u, __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_AGENT);
+        if (RG == 2) __hip_atomic_store(a.counters + kRrNotDoneWord, failed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(a.counters + kRrDoneCounter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_add(a.counters + kDecodeGenWord, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
 
-template <typename BaseT>
+template <int RG, typename BaseT>
 hipError_t launch_rr_base(const RrArgs& a, int prior_kind, int nwg, hipStream_t s) {
     const dim3 grid(nwg), block(kRrThreads);
     switch (prior_kind) {
-        case 0: hipLaunchKernelGGL((rollout_resident_kernel<BaseT, no_prior_t>), grid, block, 0, s, a); break;
-        case 1: hipLaunchKernelGGL((rollout_resident_kernel<BaseT, float>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((rollout_resident_kernel<BaseT, bf16_t>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((rollout_resident_kernel<BaseT, f16_t>), grid, block, 0, s, a); break;
+        case 0: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, no_prior_t>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, float>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, bf16_t>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, f16_t>), grid, block, 0, s, a); break;
     }
     return hipGetLastError();
+}
+
+template <int RG>
+hipError_t launch_rr(const RrArgs& a, int base_dtype, int prior_kind, int nwg, hipStream_t s) {
+    if (base_dtype == 1) return launch_rr_base<RG, bf16_t>(a, prior_kind, nwg, s);
+    if (base_dtype == 2) return launch_rr_base<RG, f16_t>(a, prior_kind, nwg, s);
+    return launch_rr_base<RG, float>(a, prior_kind, nwg, s);
 }
 
 int g_resident_spin_limit = 1 << 16;   // re-reads before a wait gives up (each ~1-2 us)
@@ -540,18 +637,21 @@ int set_rollout_resident(int enable) {
 }
 bool rollout_resident_enabled() { return g_resident_enabled != 0; }
 
-bool rollout_resident_eligible(int64_t batch, int64_t G, int64_t r, int64_t V, int64_t steps, bool packed) {
+bool rollout_resident_eligible(int64_t batch, int64_t G, int64_t r, int64_t V, int64_t steps, bool packed,
+                               size_t ws_bytes) {
     const int nwg = device_cu_count();
-    if (!packed || batch < 1 || batch > 16 || r != kResidentRank || steps < 1 || steps > kResidentMaxSteps) return false;
+    if (!packed || batch < 1 || batch > 32 || r != kResidentRank || steps < 1 || steps > kResidentMaxSteps) return false;
+    const int rg = batch > 16 ? 2 : 1;
+    if (rg == 2 && ws_bytes < kDataOff + kResident2Bytes) return false;
     if (G < 64 || G > kResidentMaxG || (G & (G - 1)) != 0 || G % nwg != 0) return false;
     // slot rows of whole 64-word chunks, at most the slots the workspace holds
     if (nwg < 64 || nwg > kResidentMaxWGs || nwg % 64 != 0 || V >= (int64_t)1 << 30) return false;
-    const int upw = (int)(G / nwg);
-    if (upw % 2 != 0 || 3 * upw > 16) return false;
+    const int upw = (int)(G / (nwg / rg));
+    if (upw % 2 != 0 || upw > 4 * rg) return false;   // up to four units (12 gate rows) per operand tile
     const int64_t ntiles = (V + 15) / 16;
-    const int64_t first = std::min<int64_t>(ntiles, (int64_t)kRrRankWGs * kRrWaves * kRrRegTiles);
-    const int64_t rest = ntiles - first;
-    const int64_t per = (rest + (nwg - kRrRankWGs) - 1) / (nwg - kRrRankWGs);
+    const int64_t first = std::min<int64_t>(ntiles, (int64_t)rg * kRrRankWGs * kRrWaves * kRrRegTiles);
+    const int64_t rest = ntiles - first, others = nwg - rg * kRrRankWGs;
+    const int64_t per = (rest + others - 1) / others;
     return per <= kRrWaves * kRrRegTiles + kResidentLdsTiles;
 }
 
@@ -569,21 +669,25 @@ hipError_t launch_rollout_resident(const ResidentRolloutArgs& r, void* ws, hipSt
     a.M = (int)r.batch; a.G = (int)r.G; a.V = (int)r.V; a.steps = (int)r.steps;
     a.ntiles = (int)((r.V + 15) / 16);
     const int nwg = device_cu_count();
-    a.upw = (int)(r.G / nwg);
+    const int rg = a.M > 16 ? 2 : 1;
+    a.upw = (int)(r.G / (nwg / rg));
     a.mp_shift = 0;
-    while ((1 << a.mp_shift) < a.M) ++a.mp_shift;
+    while ((1 << a.mp_shift) < std::min(a.M, 16)) ++a.mp_shift;
     a.np_shift = 0;
     while ((2 << a.np_shift) < a.upw) ++a.np_shift;   // upw / 2 = 1 << np_shift (upw a power of two)
     a.out_ids = r.out_ids; a.out_scores = r.out_scores; a.ld_out = r.ld_out;
     a.counters = reinterpret_cast<unsigned int*>(w + kCountersOff);
-    a.h_words = reinterpret_cast<unsigned long long*>(w + kResidentOff);
-    a.rank_words = reinterpret_cast<unsigned long long*>(w + kResidentOff + kResidentHWordBytes);
-    a.slots = reinterpret_cast<unsigned long long*>(w + kResidentOff + kResidentHWordBytes + kResidentRankWordBytes);
+    // one group: the regions that only this kernel writes; two: the data region
+    char* words = rg == 2 ? w + kDataOff : w + kResidentOff;
+    a.h_words = reinterpret_cast<unsigned long long*>(words);
+    a.rank_words = reinterpret_cast<unsigned long long*>(words + rg * kResidentHWordBytes);
+    a.slots = reinterpret_cast<unsigned long long*>(words + rg * (kResidentHWordBytes + kResidentRankWordBytes));
+    a.arrivals = reinterpret_cast<unsigned long long*>(w + kResidentOff);
     a.spin_limit = resident_spin_limit();
     const int pk = r.prior == nullptr ? 0 : (r.prior_dtype == 1 ? 2 : (r.prior_dtype == 2 ? 3 : 1));
-    if (r.base_dtype == 1) return launch_rr_base<bf16_t>(a, pk, nwg, s);
-    if (r.base_dtype == 2) return launch_rr_base<f16_t>(a, pk, nwg, s);
-    return launch_rr_base<float>(a, pk, nwg, s);
+    if (rg == 1) return launch_rr<1>(a, r.base_dtype, pk, nwg, s);
+    const hipError_t e = launch_rr<2>(a, r.base_dtype, pk, nwg, s);
+    return e != hipSuccess ? e : launch_rollout_ordered(r, ws, s);
 }
 
 }  // namespace dels

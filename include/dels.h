@@ -218,7 +218,7 @@ int dels_debug_set_decode_spin_limit(int limit);
 
 /*
  * Test hook (no counterpart in the reference).  Where the shape allows it
- * (weights in the MFMA-16 layout, r = 256, batch <= 16, G <= 1024 a multiple of
+ * (weights in the MFMA-16 layout, r = 256, batch <= 32, G <= 1024 a multiple of
  * twice the CU count, the vocabulary's share fitting a CU), dels_rollout_enqueue
  * and dels_graph_create run every step of the rollout in one launch that keeps
  * the low-rank head resident on chip, and so do the Markov rollout's entry points
@@ -230,8 +230,8 @@ int dels_debug_set_rollout_resident(int enable);
 /* Test hook: the waits of that one-launch rollout re-read each other's results
  * at most `limit` times (default 65536) before the launch gives up; a launch
  * that gives up writes -1 ids for the steps it could not finish (the Markov
- * rollout: leaves the whole rollout to the launch that follows it), and the next
- * launch starts clean.  Returns the previous limit.  Not thread-safe. */
+ * rollout, and more than 16 rows: leaves the whole rollout to the launch that
+ * follows it), and the next launch starts clean.  Returns the previous limit.  Not thread-safe. */
 int dels_debug_set_resident_spin_limit(int limit);
 
 /*
