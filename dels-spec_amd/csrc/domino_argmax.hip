@@ -19,12 +19,20 @@
 // in fp32, so the dot is that of mid to within 2^-17 relative per term -- well
 // inside the fp32 accumulation-order freedom the reference already has.
 //
-// Each workgroup builds the hi/lo operands of its 16 rows in LDS (64 * E bytes,
-// E <= 2048; rows past M are zero), then its four waves stream 16-row tiles of
-// fc2 (MFMA-16 block layout, one contiguous KiB per K step) through two
-// register sets of up to 16 K steps, walking (tile, K chunk) units so any E
-// streams with the same register budget.  The cross-workgroup argmax is the
-// GEMV kernel's (argmax_wg_finish).
+// One workgroup of eight waves per CU builds the hi/lo operands of its 16 rows
+// in LDS (64 * E bytes, E <= 2048; rows past M are zero), then its waves stream
+// 16-row tiles of fc2 (MFMA-16 block layout, one contiguous KiB per K step)
+// through two register sets of up to 16 K steps, walking (tile, K chunk) units
+// so any E streams with the same register budget.  The cross-workgroup argmax
+// is that of the other kernels (row keys and an arrival counter).
+//
+// Bound by streaming fc2 from HBM (311 MB at E = 1024, V = 151936), so the
+// stream must not start late or end in a queue: a workgroup's loads of z and s
+// go out first (a CU returns its loads in order), then the first two units of
+// every wave, and the operands are computed while those travel.  One row at
+// E = 1024, V = 151936: 65.9 -> about 54 us a launch (5.8 TB/s), the 14-step
+// rollout 1071 -> 905 us, with no waits on loads inside the stream either (see
+// EXACT) and one operand build and one arrival per CU instead of two.
 #include <algorithm>
 #include <climits>
 #include <mutex>
@@ -56,24 +64,78 @@ __device__ __forceinline__ float domino_middle(float p) {
     else return p * sigmoid_f32(p);   // DELS_MIDDLE_SILU
 }
 
-// mid = f(z + s) of the 16 rows m0 .. m0 + 15 into the hi/lo operand layout in
-// LDS (see the kernel); one loop per middle layer, so none carries a branch on it.
+constexpr int kDomWaves = 8;
+constexpr int kDomThreads = kDomWaves * 64;
+// Pieces of eight values of one row that a thread turns into operands; those
+// of E <= 1024 are held in registers while the first units are put in flight.
+constexpr int kDomPieces = 16 * 1024 / 8 / kDomThreads;
+
+// Eight values of z and s as loaded.
+struct DomPiece {
+    u32x4 z, s;
+};
+
+// z and s rows need no more than their elements' alignment: the copy states
+// that, and the compiler picks loads that are legal at it.
+__device__ __forceinline__ u32x4 load_eight(const uint16_t* p) {
+    u32x4 r;
+    __builtin_memcpy(&r, p, sizeof(r));
+    return r;
+}
+
+// Piece i: row i / (kpad / 8) of the 16, values k .. k + 7.  Rows past M and the
+// K padding are zero.
+__device__ __forceinline__ bool domino_piece_at(const DominoArgs& a, int m0, int kpad, int i, int& row, int& k) {
+    row = i / (kpad / 8);
+    k = (i - row * (kpad / 8)) * 8;
+    return m0 + row < a.M && k < a.E;
+}
+__device__ __forceinline__ void domino_load_piece(const DominoArgs& a, int m0, int kpad, int i, DomPiece& p) {
+    int row, k;
+    const bool live = i < 2 * kpad && domino_piece_at(a, m0, kpad, i, row, k);
+    // a piece without values loads the first row's first eight (in bounds) and is not used
+    const int64_t m = live ? m0 + row : m0;
+    p.z = load_eight(a.z + m * a.ldz + (live ? k : 0));
+    p.s = load_eight(a.s + m * a.lds + (live ? k : 0));
+}
+
+// mid = f(z + s) of a piece into the hi/lo operand layout in LDS (see the kernel).
 template <int MIDDLE>
-__device__ __forceinline__ void domino_fill_operands(const DominoArgs& a, int m0, int kpad, uint16_t* ops) {
+__device__ __forceinline__ void domino_store_piece(const DominoArgs& a, int m0, int kpad, int i, const DomPiece& p,
+                                                   uint16_t* ops) {
 #pragma clang fp contract(off)
-    for (int i = threadIdx.x; i < 16 * kpad; i += 256) {
-        const int row = i / kpad, k = i - row * kpad;
-        const int m = m0 + row;
-        float mid = 0.f;
-        if (m < a.M && k < a.E) {
-            const float p = bf16_bits_to_f32(a.z[(int64_t)m * a.ldz + k]) + bf16_bits_to_f32(a.s[(int64_t)m * a.lds + k]);
-            mid = domino_middle<MIDDLE>(p);
+    if (i >= 2 * kpad) return;
+    int row, k;
+    const bool live = domino_piece_at(a, m0, kpad, i, row, k);
+    u32x4 hi = {0u, 0u, 0u, 0u}, lo = {0u, 0u, 0u, 0u};
+    if (live) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int sh = 16 * (e & 1);
+            const float mid = domino_middle<MIDDLE>(bf16_bits_to_f32((p.z[e >> 1] >> sh) & 0xffffu) +
+                                                    bf16_bits_to_f32((p.s[e >> 1] >> sh) & 0xffffu));
+            const uint32_t h = f32_to_bf16_bits(mid);
+            hi[e >> 1] |= h << sh;
+            lo[e >> 1] |= (uint32_t)f32_to_bf16_bits(mid - bf16_bits_to_f32(h)) << sh;
         }
-        const uint16_t hi = f32_to_bf16_bits(mid);
-        const uint16_t lo = f32_to_bf16_bits(mid - bf16_bits_to_f32(hi));
-        const int ks = k >> 5, ln = row + 16 * ((k & 31) >> 3), e = k & 7;
-        ops[((ks * 2 + 0) * 64 + ln) * 8 + e] = hi;
-        ops[((ks * 2 + 1) * 64 + ln) * 8 + e] = lo;
+    }
+    const int ks = k >> 5, ln = row + 16 * ((k & 31) >> 3);
+    *reinterpret_cast<u32x4*>(&ops[((ks * 2 + 0) * 64 + ln) * 8]) = hi;
+    *reinterpret_cast<u32x4*>(&ops[((ks * 2 + 1) * 64 + ln) * 8]) = lo;
+}
+
+// All pieces of the workgroup: the first kDomPieces per thread from registers,
+// the rest (E > 1024) loaded here.  One instance per middle layer, so none
+// carries a branch on it.
+template <int MIDDLE>
+__device__ __forceinline__ void domino_fill_operands(const DominoArgs& a, int m0, int kpad, const DomPiece (&pc)[kDomPieces], uint16_t* ops) {
+#pragma unroll
+    for (int j = 0; j < kDomPieces; ++j)
+        domino_store_piece<MIDDLE>(a, m0, kpad, (int)threadIdx.x + kDomThreads * j, pc[j], ops);
+    for (int i = threadIdx.x + kDomThreads * kDomPieces; i < 2 * kpad; i += kDomThreads) {
+        DomPiece p;
+        domino_load_piece(a, m0, kpad, i, p);
+        domino_store_piece<MIDDLE>(a, m0, kpad, i, p, ops);
     }
 }
 
@@ -84,12 +146,15 @@ struct DomRegs {
     uint32_t bias;
 };
 
-template <typename BaseT, typename BiasT>
-__global__ __launch_bounds__(256) void domino_argmax_kernel(DominoArgs a, ArgmaxKArgs fin) {
+// EXACT: E is a whole number of register sets (a multiple of 512), so no operand
+// of fc2 is masked: a mask applied to a load would wait for it right there, and
+// the unit that is contracted meanwhile would be the only one in flight.
+template <typename BaseT, typename BiasT, bool EXACT>
+__global__ __launch_bounds__(kDomThreads) void domino_argmax_kernel(DominoArgs a, ArgmaxKArgs fin) {
 #pragma clang fp contract(off)
     extern __shared__ __attribute__((aligned(16))) char dyn_lds[];   // [ksteps][2][64 lanes][16 bytes]
-    __shared__ float s_val[4][16];
-    __shared__ int s_idx[4][16];
+    __shared__ float s_val[kDomWaves][16];
+    __shared__ int s_idx[kDomWaves][16];
     __shared__ int s_last;
 
     const int lane = threadIdx.x & 63;
@@ -106,16 +171,11 @@ __global__ __launch_bounds__(256) void domino_argmax_kernel(DominoArgs a, Argmax
     // runs every step of a set unconditionally: padded steps multiply zeros.
     uint16_t* ops = reinterpret_cast<uint16_t*>(dyn_lds);
     const int kpad = ((ksteps + kDomKC - 1) / kDomKC) * kDomKC * 32;
-    switch (a.middle) {   // uniform
-        case DELS_MIDDLE_IDENTITY: domino_fill_operands<DELS_MIDDLE_IDENTITY>(a, m0, kpad, ops); break;
-        case DELS_MIDDLE_RELU: domino_fill_operands<DELS_MIDDLE_RELU>(a, m0, kpad, ops); break;
-        case DELS_MIDDLE_GELU: domino_fill_operands<DELS_MIDDLE_GELU>(a, m0, kpad, ops); break;
-        case DELS_MIDDLE_GELU_TANH: domino_fill_operands<DELS_MIDDLE_GELU_TANH>(a, m0, kpad, ops); break;
-        case DELS_MIDDLE_TANH: domino_fill_operands<DELS_MIDDLE_TANH>(a, m0, kpad, ops); break;
-        case DELS_MIDDLE_SIGMOID: domino_fill_operands<DELS_MIDDLE_SIGMOID>(a, m0, kpad, ops); break;
-        default: domino_fill_operands<DELS_MIDDLE_SILU>(a, m0, kpad, ops); break;
-    }
-    __syncthreads();
+    DomPiece pc[kDomPieces];
+#pragma unroll
+    for (int j = 0; j < kDomPieces; ++j)
+        domino_load_piece(a, m0, kpad, (int)threadIdx.x + kDomThreads * j, pc[j]);
+    asm volatile("" ::: "memory");   // these loads stay ahead of the stream's
 
     float al[4], best[4];
     int bidx[4];
@@ -133,20 +193,25 @@ __global__ __launch_bounds__(256) void domino_argmax_kernel(DominoArgs a, Argmax
 
     const int ntiles = (a.V + 15) >> 4;
     const int nch = (ksteps + kDomKC - 1) / kDomKC;
-    const int nwaves = gridDim.x * 4;
-    const int t0 = blockIdx.x * 4 + wave;
+    const int nwaves = gridDim.x * kDomWaves;
+    const int t0 = blockIdx.x * kDomWaves + wave;
     const int cnt = t0 < ntiles ? (ntiles - 1 - t0) / nwaves + 1 : 0;
     const int units = cnt * nch;
     const BiasT* bias = static_cast<const BiasT*>(a.bias);
 
     auto load_unit = [&](int u, DomRegs<BaseT, BiasT>& tr) {
-        const int t = t0 + (u / nch) * nwaves;
+        // the first two units are loaded whether or not the wave has them (the last tile again)
+        const int t = min(t0 + (u / nch) * nwaves, ntiles - 1);
         const int c = u % nch;
         const int v = t * 16 + col;
         const int vc = v < a.V ? v : a.V - 1;
         const uint16_t* bp = a.W + ((int64_t)t * ksteps + c * kDomKC) * 512 + lane * 8;
 #pragma unroll
         for (int i = 0; i < kDomKC; ++i) {
+            if constexpr (EXACT) {
+                tr.b[i] = load_bf16x8_nt(bp + i * 512);
+                continue;
+            }
             const bool ok = c * kDomKC + i < ksteps;
             tr.b[i] = masked_bf16x8(__builtin_nontemporal_load(reinterpret_cast<const u32x4*>(bp + (ok ? i : 0) * 512)),
                                     ok ? 0xffffffffu : 0u);
@@ -184,8 +249,18 @@ __global__ __launch_bounds__(256) void domino_argmax_kernel(DominoArgs a, Argmax
     };
     // two register sets, refills unconditional inside the loop, the tail peeled
     DomRegs<BaseT, BiasT> tr0, tr1;
-    if (units > 0) load_unit(0, tr0);
-    if (units > 1) load_unit(1, tr1);
+    load_unit(0, tr0);
+    load_unit(1, tr1);
+    switch (a.middle) {   // uniform
+        case DELS_MIDDLE_IDENTITY: domino_fill_operands<DELS_MIDDLE_IDENTITY>(a, m0, kpad, pc, ops); break;
+        case DELS_MIDDLE_RELU: domino_fill_operands<DELS_MIDDLE_RELU>(a, m0, kpad, pc, ops); break;
+        case DELS_MIDDLE_GELU: domino_fill_operands<DELS_MIDDLE_GELU>(a, m0, kpad, pc, ops); break;
+        case DELS_MIDDLE_GELU_TANH: domino_fill_operands<DELS_MIDDLE_GELU_TANH>(a, m0, kpad, pc, ops); break;
+        case DELS_MIDDLE_TANH: domino_fill_operands<DELS_MIDDLE_TANH>(a, m0, kpad, pc, ops); break;
+        case DELS_MIDDLE_SIGMOID: domino_fill_operands<DELS_MIDDLE_SIGMOID>(a, m0, kpad, pc, ops); break;
+        default: domino_fill_operands<DELS_MIDDLE_SILU>(a, m0, kpad, pc, ops); break;
+    }
+    lds_barrier();   // the operands; the stream's loads stay in flight
     int u = 0;
     for (; u + 4 <= units; u += 2) {
         consume(tr0, u);
@@ -200,10 +275,10 @@ __global__ __launch_bounds__(256) void domino_argmax_kernel(DominoArgs a, Argmax
     if (u + 2 < units) consume(tr0, u + 2);
     if (u + 3 < units) consume(tr1, u + 3);
 
-    argmax_wg_finish(fin, best, bidx, m0, s_val, s_idx, s_last, nullptr);
+    argmax_wg_finish<kDomWaves>(fin, best, bidx, m0, s_val, s_idx, s_last, nullptr);
 }
 
-template <typename BaseT, typename BiasT>
+template <typename BaseT, typename BiasT, bool EXACT>
 hipError_t launch_domino_inst(const DominoArgs& a, const ArgmaxKArgs& fin, int gx, int gy, size_t lds, hipStream_t s) {
     // the operands of E = 2048 take 128 KiB of dynamic LDS: allow it once per kernel instance (the
     // attribute belongs to the function, not to a device); call_once makes concurrent first launches
@@ -211,21 +286,25 @@ hipError_t launch_domino_inst(const DominoArgs& a, const ArgmaxKArgs& fin, int g
     static std::once_flag once;
     static hipError_t attr_err = hipSuccess;
     std::call_once(once, [] {
-        attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&domino_argmax_kernel<BaseT, BiasT>),
+        attr_err = hipFuncSetAttribute(reinterpret_cast<const void*>(&domino_argmax_kernel<BaseT, BiasT, EXACT>),
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)domino_lds_bytes(kDominoMaxE));
     });
     if (attr_err != hipSuccess) return attr_err;
-    hipLaunchKernelGGL((domino_argmax_kernel<BaseT, BiasT>), dim3(gx, gy, 1), dim3(256), lds, s, a, fin);
+    hipLaunchKernelGGL((domino_argmax_kernel<BaseT, BiasT, EXACT>), dim3(gx, gy, 1), dim3(kDomThreads), lds, s, a, fin);
     return hipGetLastError();
 }
 
 template <typename BaseT>
 hipError_t launch_domino_for_base(const DominoArgs& a, const ArgmaxKArgs& fin, int gx, int gy, size_t lds,
                                   hipStream_t s) {
-    if (a.bias == nullptr) return launch_domino_inst<BaseT, no_prior_t>(a, fin, gx, gy, lds, s);
-    if (a.bias_dtype == 1) return launch_domino_inst<BaseT, bf16_t>(a, fin, gx, gy, lds, s);
-    if (a.bias_dtype == 2) return launch_domino_inst<BaseT, f16_t>(a, fin, gx, gy, lds, s);
-    return launch_domino_inst<BaseT, float>(a, fin, gx, gy, lds, s);
+    auto by_bias = [&](auto exact_tag) -> hipError_t {
+        constexpr bool EXACT = decltype(exact_tag)::value;
+        if (a.bias == nullptr) return launch_domino_inst<BaseT, no_prior_t, EXACT>(a, fin, gx, gy, lds, s);
+        if (a.bias_dtype == 1) return launch_domino_inst<BaseT, bf16_t, EXACT>(a, fin, gx, gy, lds, s);
+        if (a.bias_dtype == 2) return launch_domino_inst<BaseT, f16_t, EXACT>(a, fin, gx, gy, lds, s);
+        return launch_domino_inst<BaseT, float, EXACT>(a, fin, gx, gy, lds, s);
+    };
+    return a.E % (32 * kDomKC) == 0 ? by_bias(std::true_type{}) : by_bias(std::false_type{});
 }
 
 }  // namespace
@@ -249,11 +328,8 @@ hipError_t launch_domino_argmax(const DominoArgs& a, void* ws, hipStream_t s) {
     fin.key_stride = (int64_t)a.M * 128 <= (int64_t)(kCtrlBytes - kKeysOff) ? 16 : 1;
     const int ntiles = (a.V + 15) / 16;
     const int groups = (a.M + 15) / 16;
-    // two workgroups per CU where both fit the LDS (8 waves; the operands of E <= 1024 take 64 KiB each):
-    // 71.2 -> 69.8 us per step at 8 rows, E = 1024; more than fit at once is slower (three: 89 us)
     const size_t lds = domino_lds_bytes(a.E);
-    const int per_cu = lds <= 64 * 1024 ? 2 : 1;
-    const int gx = std::max(1, std::min((ntiles + 3) / 4, (per_cu * device_cu_count() + groups - 1) / groups));
+    const int gx = std::max(1, std::min((ntiles + kDomWaves - 1) / kDomWaves, (device_cu_count() + groups - 1) / groups));
     if (a.base_dtype == 1) return launch_domino_for_base<bf16_t>(a, fin, gx, groups, lds, s);
     if (a.base_dtype == 2) return launch_domino_for_base<f16_t>(a, fin, gx, groups, lds, s);
     return launch_domino_for_base<float>(a, fin, gx, groups, lds, s);

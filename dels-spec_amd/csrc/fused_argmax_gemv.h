@@ -108,11 +108,12 @@ __device__ __forceinline__ void load_tile(const ArgmaxKArgs& a, int t, int lane,
 
 // End of a workgroup's share of the argmax over rows m0 .. m0+15: reduce the
 // lanes' running (score, index) pairs over the 16 vocabulary columns and the
-// four waves, fold each row into its 64-bit key with a device-scope atomic max,
+// WAVES waves, fold each row into its 64-bit key with a device-scope atomic max,
 // count the workgroup in, and let the last one decode and clear the keys, the
 // counter and `also_clear` (when given).
+template <int WAVES = 4>
 __device__ __forceinline__ void argmax_wg_finish(const ArgmaxKArgs& a, float (&best)[4], int (&bidx)[4], int m0,
-                                                 float (&s_val)[4][16], int (&s_idx)[4][16], int& s_last,
+                                                 float (&s_val)[WAVES][16], int (&s_idx)[WAVES][16], int& s_last,
                                                  unsigned int* also_clear) {
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar loop control
@@ -146,7 +147,7 @@ __device__ __forceinline__ void argmax_wg_finish(const ArgmaxKArgs& a, float (&b
         float bvv = s_val[0][mi];
         int bii = s_idx[0][mi];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) {
+        for (int w = 1; w < WAVES; ++w) {
             if (argmax_better(s_val[w][mi], s_idx[w][mi], bvv, bii)) {
                 bvv = s_val[w][mi];
                 bii = s_idx[w][mi];
