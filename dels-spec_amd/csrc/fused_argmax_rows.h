@@ -9,19 +9,25 @@
 // same MFMA K steps in the same order, so scores equal the GEMV kernel's bit
 // for bit.
 //
-// Bound by streaming B from HBM once: a workgroup keeps the rank operand of RG
-// groups of 16 rows in registers (RG * r / 8 VGPRs: 256 of the 512 a wave has at
-// one wave per SIMD, for 64 rows at r = 512), so that every 16-row vocabulary
-// tile that a wave loads serves all of them, instead of being read again for
-// every 16 rows.  The tile is the MFMA's A operand and the rank its B operand:
-// lane l ends with row l % 16 of each group and the four consecutive columns
-// 4 (l / 16) .. + 3, so that a lane's base logits are one 8- or 16-byte load per
-// group, its prior values one load for all groups, and the running argmax takes
-// one (score, index) pair per group.  Streaming as in the GEMV kernel: tiles
-// walked wave-strided through two register sets, refills unconditional.
-// 40 rows, r = 512, V = 151936, bf16 base logits, whole step with its 12 us rank
-// projection: 115 us with the GEMV kernel (B read three times), 49 us here.
+// Bound by streaming B from HBM once, so every 16-row vocabulary tile that a
+// wave loads serves all the rows of its workgroup, RG groups of 16, instead of
+// being read again for every 16 rows.  The groups' rank operands lie in LDS in
+// operand order (RG * r * 32 bytes: 64 KiB for 64 rows at r = 512; each read is
+// one bank-conflict-free KiB, which feeds one MFMA: at 64 rows the LDS and the
+// matrix cores are each busy for 8 of the ~27 us the stream takes), which leaves
+// the registers to the stream: two waves per SIMD with two tiles each in flight.
+// (With the operands in registers, one wave per SIMD: 40 / 48 rows 38.5 / 39.7
+// us a launch, 33.9 / 34.7 here at r = 512, V = 151936; 64 rows of an unaligned
+// vocabulary of 50257, 37.5 and 27.1; 40 rows in the GEMV kernel, 104.)  The
+// tile is the MFMA's A operand and the rank its B operand: lane l ends with row
+// l % 16 of each group and the four consecutive columns 4 (l / 16) .. + 3, so
+// that a lane's base logits are one 8- or 16-byte load per group, its prior
+// values one load for all groups, and the running argmax takes one (score,
+// index) pair per group.  Tiles are walked wave-strided through two register
+// sets, refills unconditional, as in the GEMV kernel.
 #pragma once
+
+#include <mutex>
 
 #include "fused_argmax_gemv.h"
 #include "fused_argmax_tiled.h"
@@ -30,7 +36,8 @@ namespace dels {
 
 namespace rows {
 
-constexpr int kThreads = 256;
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * 64;
 
 // Values a lane takes from a row per tile: four consecutive ones.  VEC: as one
 // load (two words of 16-bit values, four of fp32), else four element loads.
@@ -69,12 +76,6 @@ __device__ __forceinline__ float quad_at(const uint32_t (&w)[quad_words<T, VEC>(
     else return widen_raw<T>(w[q]);
 }
 
-// Row groups per workgroup above 32 rows: 4, or 3 where the four words of base
-// logits per group and tile (fp32, or unaligned rows) leave no registers for
-// the fourth group's 64 at r = 512.
-template <int KSTEPS, typename BaseT, bool VEC>
-constexpr int max_groups() { return KSTEPS == 16 && quad_words<BaseT, VEC>() == 4 ? 3 : 4; }
-
 }  // namespace rows
 
 // Ranks the kernel takes: whole MFMA K steps, no masked operands.
@@ -87,105 +88,16 @@ struct RowsTile {
     uint32_t prior[rows::quad_words<PriorT, VEC>()];
 };
 
-// HAS_PRIOR false: the prior term is absent (PriorT is then BaseT and unused).
-template <int RG, int KSTEPS, bool ROWMAJOR, typename BaseT, typename PriorT, bool VEC, bool HAS_PRIOR>
-__global__ __launch_bounds__(rows::kThreads, 1) void fused_argmax_rows_kernel(ArgmaxKArgs a) {
-#pragma clang fp contract(off)
-    using namespace rows;
+// End of a workgroup's share of the argmax over the rows m0 .. m0 + 16 RG - 1:
+// each lane's running (score, index) pairs over the quads of columns and the
+// waves, then across workgroups.
+template <int RG>
+__device__ __forceinline__ void rows_finish(const ArgmaxKArgs& a, float (&best)[RG], int (&bidx)[RG], int m0,
+                                            float (&s_val)[rows::kWaves][16 * RG], int (&s_idx)[rows::kWaves][16 * RG],
+                                            int& s_last) {
     constexpr int kRows = 16 * RG;
-    __shared__ float s_val[4][kRows];
-    __shared__ int s_idx[4][kRows];
-    __shared__ int s_last;
-
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar loop control
-    const int col = lane & 15;     // row of the lane within each group
-    const int kg = lane >> 4;      // K octet of the operands / quad of columns of the results
-    const int m0 = blockIdx.y * kRows;
-
-    // Rank operands of the groups' rows, resident for the whole kernel; rows
-    // past M repeat row 0 (their results are not written).
-    bf16x8 ra[RG][KSTEPS];
-    float al[RG], nbe[RG], best[RG];
-    int bidx[RG];
-    bool use_prior[RG];
-    RowOff<VEC> brow[RG];
-#pragma unroll
-    for (int g = 0; g < RG; ++g) {
-        const int m = m0 + 16 * g + col;
-        const int mc = m < a.M ? m : 0;
-        const uint16_t* rp = a.rank + rank_row_of(a.rank_rows, a.rank_rows_stride, a.rank_rows_count, mc) * a.ldrank;
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) ra[g][s] = load_bf16x8(rp + s * 32 + kg * 8);
-        al[g] = a.alpha[(int64_t)mc * a.alpha_stride];
-        const float be = a.beta[(int64_t)mc * a.beta_stride];
-        nbe[g] = -be;
-        use_prior[g] = HAS_PRIOR && be != 0.f;
-        brow[g] = (RowOff<VEC>)((int64_t)mc * a.ldbase * (int64_t)sizeof(BaseT));
-        best[g] = -__builtin_inff();
-        bidx[g] = INT_MAX;
-    }
-
-    using Tile = RowsTile<RG, KSTEPS, BaseT, PriorT, VEC>;
-    auto load = [&](int t, Tile& tr) {
-        // ROWMAJOR: the lane's K octets of vocabulary row t * 16 + col; else MFMA-16 blocks
-        const uint16_t* bp = ROWMAJOR ? a.B + (int64_t)min(t * 16 + col, a.V - 1) * a.ldb + kg * 8
-                                      : a.B + (int64_t)t * (KSTEPS * 512) + lane * 8;
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s) tr.b[s] = load_bf16x8_nt(bp + s * (ROWMAJOR ? 32 : 512));
-        const int v = t * 16 + 4 * kg;
-#pragma unroll
-        for (int g = 0; g < RG; ++g) load_quad<BaseT, VEC>(a.base, brow[g], v, a.V, tr.base[g]);
-        if constexpr (HAS_PRIOR) load_quad<PriorT, VEC>(a.prior, 0, v, a.V, tr.prior);
-    };
-    auto consume = [&](const Tile& tr, int t) {
-        f32x4 acc[RG];
-#pragma unroll
-        for (int g = 0; g < RG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s = 0; s < KSTEPS; ++s)
-#pragma unroll
-            for (int g = 0; g < RG; ++g)
-                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tr.b[s], ra[g][s], acc[g], 0, 0, 0);
-        const int v = t * 16 + 4 * kg;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const bool in = v + q < a.V;
-            float pv = 0.f;
-            if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
-#pragma unroll
-            for (int g = 0; g < RG; ++g) {
-                float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT, VEC>(tr.base[g], q));
-                if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
-                // a lane's candidates arrive in increasing column order: strict ">" keeps the lowest index
-                const bool take = in & (sc > best[g]);
-                best[g] = take ? sc : best[g];
-                bidx[g] = take ? v + q : bidx[g];
-            }
-        }
-    };
-
-    // the tiles t + k * nwaves, k < cnt, through two register sets (see the GEMV kernel)
-    const int ntiles = (a.V + 15) >> 4;
-    const int nwaves = gridDim.x * 4;
-    const int t = blockIdx.x * 4 + wave;
-    const int cnt = t < ntiles ? (ntiles - 1 - t) / nwaves + 1 : 0;
-    Tile tr0, tr1;
-    if (cnt > 0) load(t, tr0);
-    if (cnt > 1) load(t + nwaves, tr1);
-    int k = 0;
-    for (; k + 4 <= cnt; k += 2) {
-        consume(tr0, t + k * nwaves);
-        load(t + (k + 2) * nwaves, tr0);
-        consume(tr1, t + (k + 1) * nwaves);
-        load(t + (k + 3) * nwaves, tr1);
-    }
-    if (k < cnt) consume(tr0, t + k * nwaves);
-    if (k + 2 < cnt) load(t + (k + 2) * nwaves, tr0);
-    if (k + 1 < cnt) consume(tr1, t + (k + 1) * nwaves);
-    if (k + 2 < cnt) consume(tr0, t + (k + 2) * nwaves);
-
-    // each row's best over the four quads of columns, then over the waves
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int col = lane & 15, kg = lane >> 4;
 #pragma unroll
     for (int g = 0; g < RG; ++g) {
 #pragma unroll
@@ -210,7 +122,7 @@ __global__ __launch_bounds__(rows::kThreads, 1) void fused_argmax_rows_kernel(Ar
         float bv = s_val[0][mi];
         int bi = s_idx[0][mi];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) {
+        for (int w = 1; w < rows::kWaves; ++w) {
             if (argmax_better(s_val[w][mi], s_idx[w][mi], bv, bi)) {
                 bv = s_val[w][mi];
                 bi = s_idx[w][mi];
@@ -222,14 +134,146 @@ __global__ __launch_bounds__(rows::kThreads, 1) void fused_argmax_rows_kernel(Ar
     tiled_argmax_finish(a, fin_m, fin_key, &s_last);
 }
 
+// HAS_PRIOR false: the prior term is absent (PriorT is then BaseT and unused).
+template <int RG, int KSTEPS, bool ROWMAJOR, typename BaseT, typename PriorT, bool VEC, bool HAS_PRIOR>
+__global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(ArgmaxKArgs a) {
+#pragma clang fp contract(off)
+    using namespace rows;
+    constexpr int kRows = 16 * RG;
+    extern __shared__ __attribute__((aligned(16))) char s_rank[];   // [KSTEPS][RG][64 lanes][16 bytes]
+    __shared__ float s_val[kWaves][kRows];
+    __shared__ int s_idx[kWaves][kRows];
+    __shared__ int s_last;
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // uniform: scalar loop control
+    const int col = lane & 15;     // row of the lane within each group
+    const int kg = lane >> 4;      // K octet of the operands / quad of columns of the results
+    const int m0 = blockIdx.y * kRows;
+
+    // Rank operands of the groups' rows, K step by K step; rows past M repeat row
+    // 0 (their results are not written).  The loads go out before the stream's.
+    constexpr int kPieces = RG * KSTEPS * 64 / kThreads;   // 16-byte pieces per thread
+    static_assert(kPieces * kThreads == RG * KSTEPS * 64, "whole pieces per thread");
+    u32x4 rp[kPieces];
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i) {
+        const int p = threadIdx.x + kThreads * i;          // piece of the LDS image: step, group, lane
+        const int l = p & 63, g = (p >> 6) % RG, s = (p >> 6) / RG;
+        const int m = m0 + 16 * g + (l & 15);
+        rp[i] = *reinterpret_cast<const u32x4*>(
+            a.rank + rank_row_of(a.rank_rows, a.rank_rows_stride, a.rank_rows_count, m < a.M ? m : 0) * a.ldrank +
+            s * 32 + (l >> 4) * 8);
+    }
+    float al[RG], nbe[RG], best[RG];
+    int bidx[RG];
+    bool use_prior[RG];
+    RowOff<VEC> brow[RG];
+#pragma unroll
+    for (int g = 0; g < RG; ++g) {
+        const int m = m0 + 16 * g + col;
+        const int mc = m < a.M ? m : 0;
+        al[g] = a.alpha[(int64_t)mc * a.alpha_stride];
+        const float be = a.beta[(int64_t)mc * a.beta_stride];
+        nbe[g] = -be;
+        use_prior[g] = HAS_PRIOR && be != 0.f;
+        brow[g] = (RowOff<VEC>)((int64_t)mc * a.ldbase * (int64_t)sizeof(BaseT));
+        best[g] = -__builtin_inff();
+        bidx[g] = INT_MAX;
+    }
+
+    using Tile = RowsTile<RG, KSTEPS, BaseT, PriorT, VEC>;
+    // live (uniform) false: not one of the wave's tiles -- the same loads, of one line each
+    auto load = [&](int t, bool live, Tile& tr) {
+        // ROWMAJOR: the lane's K octets of vocabulary row t * 16 + col; else MFMA-16 blocks
+        const uint16_t* bp = ROWMAJOR ? a.B + (int64_t)(live ? min(t * 16 + col, a.V - 1) : 0) * a.ldb + kg * 8
+                                      : a.B + (int64_t)t * (KSTEPS * 512) + (live ? lane * 8 : 0);
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) tr.b[s] = load_bf16x8_nt(bp + s * (ROWMAJOR ? 32 : 512));
+        const int v = live ? t * 16 + 4 * kg : 0;
+#pragma unroll
+        for (int g = 0; g < RG; ++g) load_quad<BaseT, VEC>(a.base, live ? brow[g] : 0, v, a.V, tr.base[g]);
+        if constexpr (HAS_PRIOR) load_quad<PriorT, VEC>(a.prior, 0, v, a.V, tr.prior);
+    };
+    auto consume = [&](const Tile& tr, int t) {
+        // the operands are read from LDS tile by tile: through the empty asm statement the
+        // compiler cannot take them for loop invariants and hold them in registers
+        int lo = lane * 16;
+        asm volatile("" : "+v"(lo));
+        f32x4 acc[RG];
+#pragma unroll
+        for (int g = 0; g < RG; ++g) acc[g] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s)
+#pragma unroll
+            for (int g = 0; g < RG; ++g)
+                acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    tr.b[s], *reinterpret_cast<const bf16x8*>(s_rank + (s * RG + g) * 1024 + lo), acc[g], 0, 0, 0);
+        const int v = t * 16 + 4 * kg;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const bool in = v + q < a.V;
+            float pv = 0.f;
+            if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
+#pragma unroll
+            for (int g = 0; g < RG; ++g) {
+                float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT, VEC>(tr.base[g], q));
+                if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
+                // a lane's candidates arrive in increasing column order: strict ">" keeps the lowest index
+                const bool take = in & (sc > best[g]);
+                best[g] = take ? sc : best[g];
+                bidx[g] = take ? v + q : bidx[g];
+            }
+        }
+    };
+
+    // the tiles t + k * nwaves, k < cnt, through two register sets (see the GEMV kernel)
+    const int ntiles = (a.V + 15) >> 4;
+    const int nwaves = gridDim.x * kWaves;
+    const int t = blockIdx.x * kWaves + wave;
+    const int cnt = t < ntiles ? (ntiles - 1 - t) / nwaves + 1 : 0;
+    Tile tr0, tr1;
+    // the first two whether or not the wave has them, so that the waits below are exact
+    load(cnt > 0 ? t : 0, cnt > 0, tr0);
+    load(cnt > 1 ? t + nwaves : 0, cnt > 1, tr1);
+#pragma unroll
+    for (int i = 0; i < kPieces; ++i)
+        *reinterpret_cast<u32x4*>(s_rank + (threadIdx.x + kThreads * i) * 16) = rp[i];
+    lds_barrier();   // the stream's loads stay in flight
+    int k = 0;
+    for (; k + 4 <= cnt; k += 2) {
+        consume(tr0, t + k * nwaves);
+        load(t + (k + 2) * nwaves, true, tr0);
+        consume(tr1, t + (k + 1) * nwaves);
+        load(t + (k + 3) * nwaves, true, tr1);
+    }
+    if (k < cnt) consume(tr0, t + k * nwaves);
+    if (k + 2 < cnt) load(t + (k + 2) * nwaves, true, tr0);
+    if (k + 1 < cnt) consume(tr1, t + (k + 1) * nwaves);
+    if (k + 2 < cnt) consume(tr0, t + (k + 2) * nwaves);
+
+    rows_finish<RG>(a, best, bidx, m0, s_val, s_idx, s_last);
+}
+
 template <int RG, int KSTEPS, bool ROWMAJOR, typename BaseT, typename PriorT, bool VEC, bool HAS_PRIOR>
 hipError_t launch_rows_inst(const ArgmaxKArgs& ka, hipStream_t s) {
     const int ntiles = (ka.V + 15) / 16;
     const int groups = (ka.M + 16 * RG - 1) / (16 * RG);
     const int cus = device_cu_count();
-    const int gx = std::max(1, std::min((ntiles + 3) / 4, (cus + groups - 1) / groups));
+    const int gx = std::max(1, std::min((ntiles + rows::kWaves - 1) / rows::kWaves, (cus + groups - 1) / groups));
+    constexpr size_t kLds = (size_t)RG * KSTEPS * 1024;
+    // more than 64 KiB of dynamic LDS is allowed once per kernel instance (see launch_domino_inst)
+    static std::once_flag once;
+    static hipError_t attr_err = hipSuccess;
+    std::call_once(once, [] {
+        attr_err = hipFuncSetAttribute(
+            reinterpret_cast<const void*>(
+                &fused_argmax_rows_kernel<RG, KSTEPS, ROWMAJOR, BaseT, PriorT, VEC, HAS_PRIOR>),
+            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
+    });
+    if (attr_err != hipSuccess) return attr_err;
     hipLaunchKernelGGL((fused_argmax_rows_kernel<RG, KSTEPS, ROWMAJOR, BaseT, PriorT, VEC, HAS_PRIOR>),
-                       dim3(gx, groups, 1), dim3(rows::kThreads), 0, s, ka);
+                       dim3(gx, groups, 1), dim3(rows::kThreads), kLds, s, ka);
     return hipGetLastError();
 }
 
@@ -254,7 +298,16 @@ hipError_t launch_rows_for_base(const ArgmaxKArgs& ka, bool packed, int prior_ki
             constexpr int KS = decltype(ks_tag)::value;
             constexpr bool RM = decltype(rm_tag)::value;
             if (ka.M <= 32) return launch_rows_inst<2, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
-            return launch_rows_inst<rows::max_groups<KS, BaseT, VEC>(), KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+            // three groups where their operands split evenly over the threads; eight, past
+            // 64 rows, where their base logits fit the registers (200 rows, row-major:
+            // 141 us with four, 114 with eight)
+            if constexpr (VEC) {
+                if constexpr (KS >= 8)
+                    if (ka.M <= 48) return launch_rows_inst<3, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+                if constexpr (sizeof(BaseT) == 2)
+                    if (ka.M > 64) return launch_rows_inst<8, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+            }
+            return launch_rows_inst<4, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
         };
         auto by_layout = [&](auto ks_tag) -> hipError_t {
             return packed ? by_rows(ks_tag, False{}) : by_rows(ks_tag, True{});
