@@ -1018,7 +1018,7 @@ int dels_lowrank_argmax_fp8(const void* h, int64_t ldh, const void* Aq, const fl
         e = launch_lowrank_decode(ra, a, ws, s);
         return e == hipSuccess ? DELS_OK : hip_fail(e, "fp8 fused decode step launch");
     }
-    if (fp8_argmax_tiled(a) && rank_proj_quantizes(L.plan, r)) {
+    if (fp8_argmax_tiled(a) && rank_proj_quantizes(L.plan, ra)) {
         // the rank epilogue also writes the rank quantised per row where the
         // e4m3 tiled argmax reads it: no quantisation launch
         ra.rank_q = reinterpret_cast<uint8_t*>(w + L.argmax_off);

@@ -61,8 +61,11 @@ constexpr size_t kDataOff = kResidentOff + kResidentWordBytes;
 
 // ---- skinny GEMM: rank projection and fused GRU step -----------------------
 
-// Rows from which the rank projection uses the LDS-tiled kernel.
-constexpr int kRankTiledMinRows = 64;
+// Rows from which the rank projection uses the LDS-tiled kernel, and up to
+// kRankWholeK from kRankTiledMinRowsShortK rows on (see plan_skinny).
+constexpr int kRankTiledMinRows = 17;
+constexpr int kRankTiledMinRowsShortK = 64;
+constexpr int kRankWholeK = 2048;
 
 struct SkinnyPlan {
     bool tiled;        // rank projection by the LDS-tiled kernel (many rows)
@@ -94,7 +97,7 @@ struct RankArgs {
 };
 // Whether launch_rank_proj with plan p can also write the rank quantised per
 // row to e4m3 (the LDS-tiled GEMM with split K, r = 256 or 512).
-bool rank_proj_quantizes(const SkinnyPlan& p, int64_t r);
+bool rank_proj_quantizes(const SkinnyPlan& p, const RankArgs& a);
 // `ws` is the workspace base (control area); partials go to ws + data_off.
 hipError_t launch_rank_proj(const RankArgs& a, const SkinnyPlan& p, void* ws, size_t data_off, hipStream_t s);
 

@@ -303,7 +303,7 @@ __global__ __launch_bounds__(256) void skinny_gemm_kernel(SkinnyKArgs a) {
 }
 
 // ---------------------------------------------------------------------------
-// Many rows (M >= 64): an LDS-tiled rank projection.
+// Many rows (17 and more, plan_skinny): an LDS-tiled rank projection.
 //
 // The skinny kernel reads its operands straight from global memory, each
 // wave's load touching 32 B of 32 different rows; at M = 512 that re-reads h
@@ -601,7 +601,18 @@ __global__ __launch_bounds__(256) void rank_splitk_epilogue_kernel(SkinnyKArgs a
     }
 }
 
-bool rank_proj_quantizes(const SkinnyPlan& p, int64_t r) { return p.tiled && p.ksplit > 1 && (r == 256 || r == 512); }
+// The tiled kernel's 32-bit byte offsets from a tile's first row reach all of
+// its rows; wider views (a leading dimension of millions) and hidden sizes take
+// the skinny kernel, with K whole.
+static bool rank_tiled_offsets_ok(const RankArgs& a) {
+    const int64_t lim = (int64_t)1 << 32;
+    if ((128 * a.ldh + a.d) * 2 >= lim) return false;
+    return a.a_packed || a.a_scale ? a.d < (int64_t)1 << 25 : (64 * a.lda + a.d) * 2 < lim;
+}
+
+bool rank_proj_quantizes(const SkinnyPlan& p, const RankArgs& a) {
+    return p.tiled && p.ksplit > 1 && (a.r == 256 || a.r == 512) && rank_tiled_offsets_ok(a);
+}
 
 // ---------------------------------------------------------------------------
 // Host side
@@ -611,14 +622,21 @@ static inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
 SkinnyPlan plan_skinny(int64_t rows, int64_t K, int64_t cols, bool gru) {
     SkinnyPlan p{};
-    if (!gru && rows >= kRankTiledMinRows && K % kRgChunk == 0 && cols % 8 == 0) {
+    const int tiled_rows = K > kRankWholeK ? kRankTiledMinRows : kRankTiledMinRowsShortK;
+    if (!gru && rows >= tiled_rows && K % kRgChunk == 0 && cols % 8 == 0) {
         // LDS-tiled kernel.  Tiles of 128 rows x 64 columns from 256 rows on
         // (64 x 64 below, where a 128-row tile would be mostly empty), K split
-        // 8 ways unless the tiles alone fill the device, never below two chunks
-        // per split.  At M = 512, r = 512, d = 4096 the shapes measured (GEMM
-        // kernel, rocprof average): 64x64 / 8 splits 9.45 us, 128x64 / 8 8.89,
-        // 128x128 / 16 10.44 (twice the partials), with the split-K epilogue
-        // 4.9-5.2 us in each case.
+        // 8 ways unless the tiles alone fill the device, 16 ways up to 32 rows (no
+        // more partials than 64 rows in 8 splits), never below two chunks per
+        // split.  From 17 rows on where K is long: d = 4096, r = 512, 17 / 40 rows
+        // 12.5 / 11.1 us in the skinny kernel (whose splits meet in device-coherent
+        // partials), 8.0 / 9.0 here; d = 2560, r = 256, 10.9 / 12.3 against 7.5 /
+        // 7.8.  Up to d = 2048 the skinny kernel keeps K whole in one launch
+        // and is as good below 64 rows (d = 1024: 5.7 - 6.6 against 6.6 - 7.2; d =
+        // 2048: 7.3 - 10.2 against 7.4 - 8.3).
+        // At M = 512, r = 512, d = 4096 the shapes measured (GEMM kernel, rocprof
+        // average): 64x64 / 8 splits 9.45 us, 128x64 / 8 8.89, 128x128 / 16 10.44
+        // (twice the partials), with the split-K epilogue 4.9-5.2 us in each case.
         p.tiled = true;
         p.wm = p.wn = 0;
         p.tm = rows >= 256 ? 128 : 64;
@@ -628,10 +646,12 @@ SkinnyPlan plan_skinny(int64_t rows, int64_t K, int64_t cols, bool gru) {
         p.ksteps = (int)cdiv(K, 32);
         const int nchunks = (int)(K / kRgChunk);
         const int tiles = p.m_wg * p.n_wg;
-        int ks = tiles >= 256 ? 1 : 8;
+        int ks = tiles >= 256 ? 1 : rows <= 32 ? 16 : 8;
         ks = std::min(ks, std::max(1, nchunks / 2));
         p.ksplit = std::min(ks, kMaxKSplit);
-        p.partial_bytes = p.ksplit > 1 ? (size_t)p.ksplit * rows * cols * sizeof(float) : 0;
+        // (never less than 64 rows' 8 splits: a workspace made for more rows serves fewer)
+        const int64_t prows = std::max<int64_t>(p.ksplit * rows, rows < kRankTiledMinRowsShortK ? 512 : 0);
+        p.partial_bytes = p.ksplit > 1 ? (size_t)prows * cols * sizeof(float) : 0;
         return p;
     }
     if (gru) {
@@ -708,6 +728,14 @@ hipError_t launch_rank_proj(const RankArgs& a, const SkinnyPlan& p, void* ws, si
     ka.out = a.rank; ka.ldout = a.ldrank;
     fill_ws(ka, p, ws, data_off);
     const int wmode = a.a_scale ? W_PACKED_E4M3 : (a.a_packed ? W_PACKED : W_ROWMAJOR);
+    if (p.tiled && !rank_tiled_offsets_ok(a)) {
+        SkinnyPlan q = p;
+        q.wm = q.wn = 2;
+        q.m_wg = (int)cdiv(a.M, 32);
+        q.n_wg = (int)cdiv(a.r, 32);
+        q.ksplit = ka.ksplit = 1;
+        return launch_skinny<2, 2, EPI_RANK>(ka, q, wmode, s);
+    }
     if (p.tiled) {
         const dim3 grid(p.ksplit, p.n_wg, p.m_wg);
         hipError_t e0 = hipSuccess;
@@ -720,7 +748,7 @@ hipError_t launch_rank_proj(const RankArgs& a, const SkinnyPlan& p, void* ws, si
         const int64_t quads = (int64_t)ka.M * ka.ncols / 4;
         const dim3 egrid((unsigned)((quads + 255) / 256));
         if (a.rank_q != nullptr) {
-            if (!rank_proj_quantizes(p, a.r)) return hipErrorInvalidValue;
+            if (!rank_proj_quantizes(p, a)) return hipErrorInvalidValue;
             ka.out_q = a.rank_q;
             ka.out_qscale = a.rank_qscale;
             hipLaunchKernelGGL(rank_splitk_epilogue_kernel<true>, egrid, dim3(256), 0, s, ka);
