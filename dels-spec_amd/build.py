@@ -21,7 +21,8 @@ LIB_PATH = os.path.join(LIB_DIR, LIB_NAME)
 
 SOURCES = ["capi.hip", "skinny_gemm.hip", "fused_argmax.hip", "fused_argmax_f32.hip", "fused_argmax_bf16.hip",
            "fused_argmax_f16.hip", "fused_argmax_rows_f32.hip", "fused_argmax_rows_bf16.hip",
-           "fused_argmax_rows_f16.hip", "fused_argmax_tiled_f32.hip", "fused_argmax_tiled_bf16.hip",
+           "fused_argmax_rows_f16.hip", "fused_argmax_rows8_f32.hip", "fused_argmax_rows8_bf16.hip",
+           "fused_argmax_rows8_f16.hip", "fused_argmax_tiled_f32.hip", "fused_argmax_tiled_bf16.hip",
            "fused_argmax_tiled_f16.hip", "lowrank_decode_f32.hip", "lowrank_decode_bf16.hip",
            "lowrank_decode_f16.hip", "pack.hip", "sample.hip", "domino_argmax.hip", "lm_head.hip",
            "rollout_resident.hip", "markov_resident.hip", "rollout_ordered.hip"]

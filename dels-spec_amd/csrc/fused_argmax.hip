@@ -7,6 +7,7 @@
 #include "fused_argmax_fp8.h"
 #include "fused_argmax_gemv.h"
 #include "fused_argmax_rows.h"
+#include "fused_argmax_rows8.h"
 #include "fused_argmax_tiled.h"
 #include "fused_argmax_tiled8.h"
 #include "lowrank_decode.h"
@@ -331,6 +332,11 @@ static bool tiled8_eligible(const ArgmaxArgs& a) {
 
 bool fp8_argmax_tiled(const ArgmaxArgs& a) { return tiled8_eligible(a); }
 
+// Four-element loads also of the B scales.
+static bool rows8_vec(const ArgmaxArgs& a) {
+    return rows_vec(a) && (reinterpret_cast<uintptr_t>(a.b_scale) & 15) == 0;
+}
+
 hipError_t launch_fused_argmax_fp8(const ArgmaxArgs& a, void* ws, size_t data_off, hipStream_t s) {
     const int pk = a.prior == nullptr ? 0 : (a.prior_dtype == 1 ? 2 : (a.prior_dtype == 2 ? 3 : 1));
     char* w = static_cast<char*>(ws);
@@ -382,6 +388,12 @@ hipError_t launch_fused_argmax_fp8(const ArgmaxArgs& a, void* ws, size_t data_of
     ka.counter = reinterpret_cast<unsigned int*>(w + kCountersOff);
     ka.keys = reinterpret_cast<unsigned long long*>(w + kKeysOff);
     ka.key_stride = (int64_t)a.M * 128 <= (int64_t)(kCtrlBytes - kKeysOff) ? 16 : 1;
+    if (a.M >= kRowsMinRows && rows8_rank_ok(a.r) && rows_prior_ok(a.base_dtype, pk)) {
+        const bool vec = rows8_vec(a);
+        if (a.base_dtype == 1) return launch_rows8_bf16(ka, pk, vec, s);
+        if (a.base_dtype == 2) return launch_rows8_f16(ka, pk, vec, s);
+        return launch_rows8_f32(ka, pk, vec, s);
+    }
     if (a.base_dtype == 1) return launch_gemv8_bf16(ka, pk, s);
     if (a.base_dtype == 2) return launch_gemv8_f16(ka, pk, s);
     return launch_gemv8_f32(ka, pk, s);
