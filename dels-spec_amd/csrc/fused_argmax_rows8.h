@@ -11,9 +11,12 @@
 // 32 KiB for 64 rows at r = 512); a tile is half of the bf16 kernel's registers,
 // so three of them per wave are in flight at two waves per SIMD.  The GEMV
 // kernel that this replaces reads B once per 16 rows.  r = 512, V = 151936, bf16
-// base logits: 24 rows 24.1 -> 22.3 us, 40 rows 63.7 -> 27.9, 56 rows 38.6 ->
-// 29.0; 200 rows of an unaligned vocabulary of 50257, 74.6 -> 58.6.  (At 96 rows a variant
-// with eight groups took 41 us where the tiled kernel takes 30: not kept.)
+// base logits: 24 rows 23.8 -> 21.1 us, 40 rows 62.9 -> 26.6; V = 32000, 40 rows
+// 20.1 -> 14.5; r = 256, V = 65536, 40 / 63 rows 16.4 / 18.7 -> 14.8 / 15.5, and
+// V = 32000, 40 rows 12.3 -> 12.8, the one size measured that gained nothing;
+// 200 rows of an unaligned vocabulary of 50257, 74.6 -> 58.6.  (Above 63
+// rows aligned rows go to the tiled kernel: 96 rows 30 us there, 41 in a variant
+// of this one with eight groups.)
 #pragma once
 
 #include <mutex>
