@@ -11,13 +11,12 @@
 // its base logits, the rank rows and one slot word per row and workgroup.
 // What bounds a step is the chain: publish the slot words, read everyone's,
 // gather the embedding rows they name, contract, publish.  14 steps of 4 rows at
-// V = 151936, r = 256, with the copies of a runner's call: 279.6 -> 118.6 us.
+// V = 151936, r = 256, with the copies of a runner's call: 279.6 -> 107.9 us.
 //
 //   * argmax: every wave contracts its resident tiles against the rank of up
-//     to two groups of 16 rows (v_mfma_f32_16x16x32_bf16, lane l holding rows
-//     4(l/16)+q of column l%16), combines s = fma(-beta, prior, fma(dot,
-//     alpha, base)) as every kernel of the path does, and the workgroup
-//     publishes each row's best as one slot word (rr_slot_maxima);
+//     to two groups of 16 rows and combines s = fma(-beta, prior, fma(dot,
+//     alpha, base)) as every kernel of the path does (rr_tiles_best), and the
+//     workgroup publishes each row's best as one slot word (rr_slot_maxima);
 //   * every workgroup reads all slots of each row, takes the maximum, and so
 //     knows the step's ids, whose embedding rows it loads into LDS.
 //
@@ -38,14 +37,14 @@ namespace {
 
 constexpr int kMrPad = 8;   // bf16 of padding per rank row in LDS (rows 16 B apart in banks)
 
-template <int RG, int KS, typename BaseT, typename PriorT>
+template <int RG, int KS, typename BaseT, typename PriorT, bool VEC>
 __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRolloutArgs a) {
 #pragma clang fp contract(off)
     constexpr int kRows = 16 * RG;
     constexpr int kPitch = KS * 32 + kMrPad;
     __shared__ __attribute__((aligned(16))) char s_b[kResidentLdsTiles * KS * 1024];
     __shared__ __attribute__((aligned(16))) uint16_t s_rank[kRows * kPitch];
-    __shared__ float s_prior[(kRrWaves * kRrRegTiles + kResidentLdsTiles) * 16];
+    __shared__ __attribute__((aligned(16))) float s_prior[kRrPriorWords];
     __shared__ unsigned long long s_key[kRrWaves][kRows];   // each wave's best key of each row
     __shared__ unsigned long long s_rowmax[kRows];          // the step's maximum slot word of each row
     __shared__ float s_ab[2][kResidentMaxSteps];
@@ -94,6 +93,7 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
         *reinterpret_cast<u32x4*>(s_b + (e * KS + s) * 1024 + l * 16) =
             *reinterpret_cast<const u32x4*>(a.B + ((int64_t)t * KS + s) * 512 + l * 8);
     }
+    if (threadIdx.x < 16) s_prior[kRrPriorZeros + threadIdx.x] = 0.f;
     for (int i = threadIdx.x; i < ntl * 16; i += kRrThreads) {
         const int v = min(T0 * 16 + i, V - 1);
         if constexpr (is_no_prior<PriorT>::value) s_prior[i] = 0.f;
@@ -143,22 +143,12 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
             t = t < 0 ? 0 : (t >= a.table_rows ? a.table_rows - 1 : t);
             rp[i] = *reinterpret_cast<const u32x4*>(a.embedding + t * a.ld_embedding + (p - m * kPieces) * 8);
         }
-        uint32_t braw[RG][kRrRegTiles + 1][4];
-        {
-            const BaseT* bs = base + (int64_t)s * V;
+        RrBase<BaseT> braw[RG];
 #pragma unroll
-            for (int g = 0; g < RG; ++g)
-#pragma unroll
-                for (int j = 0; j <= kRrRegTiles; ++j) {
-                    const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
-                    const int tc = min(T0 + min(ti, max(ntl - 1, 0)), a.ntiles - 1);
-                    const int vc = min(tc * 16 + lcol, V - 1);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int m = 16 * g + 4 * lkg + q;
-                        braw[g][j][q] = load_raw(bs + (int64_t)(m < M ? m : 0) * a.ld_base + vc);
-                    }
-                }
+        for (int g = 0; g < RG; ++g) {
+            const int m = 16 * g + lcol;
+            rr_load_base<BaseT, VEC>(base + (int64_t)s * V + (int64_t)(m < M ? m : 0) * a.ld_base, T0, ntl, a.ntiles,
+                                     wave, lkg, V, braw[g]);
         }
         asm volatile("" ::: "memory");   // the base loads are issued before the rank rows are waited for
 #pragma unroll
@@ -169,60 +159,14 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
         }
         __syncthreads();
 
-        const float al = s_ab[0][s], be = s_ab[1][s];
-        const bool use_prior = !is_no_prior<PriorT>::value && be != 0.f;
         const bool lds_tile = wave < nlds;
-        const int lslot = lds_tile ? wave : 0;
+        const char* ltile = s_b + (lds_tile ? wave : 0) * KS * 1024;
 #pragma unroll
         for (int g = 0; g < RG; ++g) {
-            f32x4 acc[kRrRegTiles + 1];
-#pragma unroll
-            for (int j = 0; j <= kRrRegTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            // unconditional contractions (no branches between the MFMAs): a tile
-            // that is not this wave's is not combined
-#pragma unroll
-            for (int k = 0; k < KS; ++k) {
-                const bf16x8 rk =
-                    *reinterpret_cast<const bf16x8*>(&s_rank[(16 * g + lcol) * kPitch + k * 32 + lkg * 8]);
-                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(s_b + (lslot * KS + k) * 1024 + lane * 16);
-#pragma unroll
-                for (int j = 0; j < kRrRegTiles; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bt[j][k], acc[j], 0, 0, 0);
-                acc[kRrRegTiles] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bv, acc[kRrRegTiles], 0, 0, 0);
-            }
-            float best[4];
-            int bidx[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { best[q] = -__builtin_inff(); bidx[q] = INT_MAX; }
-            // a lane's column grows with its tile number, so a later tile takes
-            // the lead only on a larger score
-#pragma unroll
-            for (int j = 0; j <= kRrRegTiles; ++j) {
-                const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
-                const bool live = j < kRrRegTiles ? ti < ntl : lds_tile;   // wave-uniform
-                const int tc = min(ti, max(ntl - 1, 0));
-                const int v = (T0 + tc) * 16 + lcol;
-                const bool livev = live & (v < V);
-                const float pv = s_prior[tc * 16 + lcol];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float sc = __builtin_fmaf(acc[j][q], al, widen_raw<BaseT>(braw[g][j][q]));
-                    if (use_prior) sc = __builtin_fmaf(-be, pv, sc);
-                    const bool take = livev & (sc > best[q]);
-                    best[q] = take ? sc : best[q];
-                    bidx[q] = take ? v : bidx[q];
-                }
-            }
-            // over the 16 columns of each row as argmax keys (lane 15 of a DPP row ends with the row's best)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                unsigned long long key = pack_argmax(best[q], (uint32_t)bidx[q]);
-                rr_row_max<1>(key);
-                rr_row_max<2>(key);
-                rr_row_max<4>(key);
-                rr_row_max<8>(key);
-                if (col == 15) s_key[wave][16 * g + 4 * kg + q] = key;
-            }
+            const unsigned long long key = rr_tiles_best<KS, false, BaseT, PriorT, VEC>(
+                bt, ltile, lds_tile, &s_rank[(16 * g + lcol) * kPitch + lkg * 8], braw[g], s_prior, T0, ntl, wave, lkg,
+                V, s_ab[0][s], s_ab[1][s]);
+            if (kg == 0) s_key[wave][16 * g + col] = key;
         }
         __syncthreads();
         // the workgroup's best of each row into its slot word for the step
@@ -288,23 +232,29 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
     __hip_atomic_fetch_add(a.counters + kDecodeGenWord, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <int RG, int KS, typename BaseT>
+template <int RG, int KS, typename BaseT, bool VEC>
 hipError_t launch_mr(const MarkovRolloutArgs& a, int prior_kind, int nwg, hipStream_t s) {
     const dim3 grid(nwg), block(kRrThreads);
     switch (prior_kind) {
-        case 0: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, no_prior_t>), grid, block, 0, s, a); break;
-        case 1: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, float>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, bf16_t>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, f16_t>), grid, block, 0, s, a); break;
+        case 0: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, no_prior_t, VEC>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, float, VEC>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, bf16_t, VEC>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((markov_resident_kernel<RG, KS, BaseT, f16_t, VEC>), grid, block, 0, s, a); break;
     }
     return hipGetLastError();
 }
 
 template <typename BaseT>
 hipError_t launch_mr_base(const MarkovRolloutArgs& a, int prior_kind, int nwg, hipStream_t s) {
-    if (a.r == 256)
-        return a.M <= 16 ? launch_mr<1, 8, BaseT>(a, prior_kind, nwg, s) : launch_mr<2, 8, BaseT>(a, prior_kind, nwg, s);
-    return a.M <= 16 ? launch_mr<1, 4, BaseT>(a, prior_kind, nwg, s) : launch_mr<2, 4, BaseT>(a, prior_kind, nwg, s);
+    auto by_shape = [&](auto vec) -> hipError_t {
+        constexpr bool VEC = decltype(vec)::value;
+        if (a.r == 256)
+            return a.M <= 16 ? launch_mr<1, 8, BaseT, VEC>(a, prior_kind, nwg, s)
+                             : launch_mr<2, 8, BaseT, VEC>(a, prior_kind, nwg, s);
+        return a.M <= 16 ? launch_mr<1, 4, BaseT, VEC>(a, prior_kind, nwg, s)
+                         : launch_mr<2, 4, BaseT, VEC>(a, prior_kind, nwg, s);
+    };
+    return rr_vec(a.base, a.base_dtype, a.ld_base, a.V) ? by_shape(std::true_type{}) : by_shape(std::false_type{});
 }
 
 }  // namespace

@@ -8,6 +8,7 @@
 
 #include "dels_device.h"
 #include "dels_internal.h"
+#include "fused_argmax_rows.h"
 
 namespace dels {
 
@@ -172,6 +173,163 @@ __device__ __forceinline__ void rr_row_max(unsigned long long& k) {
     const uint32_t hi = (uint32_t)__builtin_amdgcn_mov_dpp((int)(uint32_t)(k >> 32), kRowShr, 0xf, 0xf, true);
     const unsigned long long o = ((unsigned long long)hi << 32) | lo;
     k = o > k ? o : k;
+}
+
+// The prior in LDS: a float per column of the workgroup's tiles, then a tile of zeros.
+constexpr int kRrPriorZeros = (kRrWaves * kRrRegTiles + kResidentLdsTiles) * 16;
+constexpr int kRrPriorWords = kRrPriorZeros + 16;
+
+// Base logits of the wave's tiles for one group of 16 rows: lane (col, kg) takes
+// row `col` of the group, columns 4 kg .. 4 kg + 3 of each tile, as one 8- or
+// 16-byte load per tile.  VEC: V and the row stride multiples of four, the base
+// aligned to four elements.  (Element loads take a line per row each: twenty of
+// them per lane and group made a vocabulary of 50257 slower than one of 151936.)
+template <typename BaseT>
+using RrQuad = uint32_t[rows::quad_words<BaseT, true>()];
+template <typename BaseT>
+using RrBase = RrQuad<BaseT>[kRrRegTiles + 1];
+
+// `row`: the lane's row of the step.  Tiles past the workgroup's repeat its last one.
+template <typename BaseT, bool VEC>
+__device__ __forceinline__ void rr_load_base(const BaseT* row, int T0, int ntl, int ntiles, int wave, int kg, int V,
+                                             RrBase<BaseT>& w) {
+#pragma unroll
+    for (int j = 0; j <= kRrRegTiles; ++j) {
+        const int tc = min(T0 + min(wave + 8 * j, max(ntl - 1, 0)), ntiles - 1);
+        const int v = tc * 16 + 4 * kg;
+        if constexpr (VEC) {
+            const BaseT* p = row + min(v, V - 4);
+            if constexpr (sizeof(BaseT) == 2) {
+                const u32x2 x = *reinterpret_cast<const u32x2*>(p);
+                w[j][0] = x[0]; w[j][1] = x[1];
+            } else {
+                const u32x4 x = *reinterpret_cast<const u32x4*>(p);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[j][q] = x[q];
+            }
+        } else if (V >= 4) {
+            // elsewhere a quad is one load at element alignment, taken back into the
+            // row at its end (rr_shift_quad puts its elements in place when it is used)
+            const BaseT* p = row + min(v, V - 4);
+            if constexpr (sizeof(BaseT) == 2) {
+                typedef uint64_t __attribute__((aligned(2))) u64_a2;
+                const uint64_t x = *reinterpret_cast<const u64_a2*>(p);
+                w[j][0] = (uint32_t)x; w[j][1] = (uint32_t)(x >> 32);
+            } else {
+                typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+                const u32x4 x = *reinterpret_cast<const u32x4_a4*>(p);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[j][q] = x[q];
+            }
+        } else {
+            uint32_t e[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) e[q] = load_raw(row + min(v + q, V - 1));
+            if constexpr (sizeof(BaseT) == 2) {
+                w[j][0] = (e[0] & 0xffffu) | e[1] << 16;
+                w[j][1] = (e[2] & 0xffffu) | e[3] << 16;
+            } else {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) w[j][q] = e[q];
+            }
+        }
+    }
+}
+
+// The quad of columns v .. v + 3 from one that was taken back to V - 4 (columns
+// past V are not used).
+template <typename BaseT>
+__device__ __forceinline__ void rr_shift_quad(RrQuad<BaseT>& w, int v, int V) {
+    const int d = V >= 4 ? min(max(v - (V - 4), 0), 3) : 0;
+    if constexpr (sizeof(BaseT) == 2) {
+        const uint64_t x = (((uint64_t)w[1] << 32) | w[0]) >> (16 * d);
+        w[0] = (uint32_t)x; w[1] = (uint32_t)(x >> 32);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int o = 1; q + o < 4; ++o) w[q] = d == o ? w[q + o] : w[q];
+    }
+}
+
+// The wave's best of one group of 16 rows over its resident tiles (register
+// tile j: vocabulary tile T0 + wave + 8 j; the LDS tile at `ltile`, vocabulary
+// tile T0 + 32 + wave, when lds_tile) as an argmax key, valid in lanes 0 .. 15
+// for row `lane` of the group.  The tile is the MFMA's A operand and the rank
+// (`rank`: the lane's first octet of row `col`) its B operand, so that lane
+// (col, kg) ends with row col and the four consecutive columns 4 kg ..: one quad
+// load of base logits per tile, one (score, candidate) pair per lane and two
+// exchanges across lanes.  (The other way round a lane holds four rows of one
+// column: twenty 2-byte loads, four pairs and sixteen exchanges.)  K step
+// outermost: each rank operand is read from LDS once and feeds every tile; no
+// branches between the MFMAs: a tile that is not the wave's is not combined.
+// TAKE_INF: a row whose best score is -inf names its first column at that score.
+template <int KS, bool TAKE_INF, typename BaseT, typename PriorT, bool VEC>
+__device__ __forceinline__ unsigned long long rr_tiles_best(const bf16x8 (&bt)[kRrRegTiles][KS], const char* ltile,
+                                                            bool lds_tile, const uint16_t* rank,
+                                                            RrBase<BaseT>& braw, const float* s_prior,
+                                                            int T0, int ntl, int wave, int kg, int V, float al,
+                                                            float be) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    f32x4 acc[kRrRegTiles + 1];
+#pragma unroll
+    for (int j = 0; j <= kRrRegTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < KS; ++k) {
+        const bf16x8 rk = *reinterpret_cast<const bf16x8*>(rank + k * 32);
+        const bf16x8 bv = *reinterpret_cast<const bf16x8*>(ltile + k * 1024 + lane * 16);
+#pragma unroll
+        for (int j = 0; j < kRrRegTiles; ++j)
+            acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bt[j][k], rk, acc[j], 0, 0, 0);
+        acc[kRrRegTiles] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bv, rk, acc[kRrRegTiles], 0, 0, 0);
+    }
+    asm volatile("" ::: "memory");   // the prior is read now: held from before the contraction it costs spills
+    // Scores in place of the sums.  A column that is not there scores NaN (through
+    // its alpha), which neither the maximum nor the comparison takes; beta 0 reads
+    // the zeros behind the prior, and fma(-0, 0, s) is s.
+    const float nan = __builtin_nanf("");
+    float best = -__builtin_inff();
+#pragma unroll
+    for (int j = 0; j <= kRrRegTiles; ++j) {
+        const int ti = wave + 8 * j;
+        const bool live = j < kRrRegTiles ? ti < ntl : lds_tile;   // wave-uniform
+        const int tc = min(ti, max(ntl - 1, 0));
+        const int left = live ? V - (T0 + tc) * 16 - 4 * kg : 0;   // columns from the lane's first one on
+        if constexpr (!VEC)
+            if ((T0 + tc) * 16 + 16 > V) rr_shift_quad<BaseT>(braw[j], (T0 + tc) * 16 + 4 * kg, V);   // wave-uniform
+        f32x4 pv = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (!is_no_prior<PriorT>::value)
+            pv = *reinterpret_cast<const f32x4*>(s_prior + (be != 0.f ? tc * 16 : kRrPriorZeros) + 4 * kg);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float al_q = (VEC ? 0 : q) < left ? al : nan;
+            float sc = __builtin_fmaf(acc[j][q], al_q, rows::quad_at<BaseT, true>(braw[j], q));
+            if constexpr (!is_no_prior<PriorT>::value) sc = __builtin_fmaf(-be, pv[q], sc);
+            acc[j][q] = sc;
+            best = __builtin_fmaxf(best, sc);
+        }
+    }
+    // the lowest of the lane's columns at its maximum, which grow with 4 j + q
+    int cand = -1;
+#pragma unroll
+    for (int c = 4 * kRrRegTiles + 3; c >= 0; --c) cand = acc[c >> 2][c & 3] == best ? c : cand;
+    if constexpr (!TAKE_INF) cand = best == -__builtin_inff() ? -1 : cand;
+    // candidate 4 j + q is column (T0 + wave + 8 j) * 16 + 4 kg + q; none: INT_MAX
+    const int idx = cand < 0 ? INT_MAX : (T0 + wave + 8 * (cand >> 2)) * 16 + 4 * kg + (cand & 3);
+    unsigned long long key = pack_argmax(best, (uint32_t)idx);
+#pragma unroll
+    for (int off = 16; off < 64; off <<= 1) {
+        const unsigned long long o = __shfl_xor(key, off, 64);
+        key = o > key ? o : key;
+    }
+    return key;
+}
+
+// Whether quads of base logits can be loaded as one.
+inline bool rr_vec(const void* base, int base_dtype, int64_t ld_base, int64_t V) {
+    const uintptr_t align = base_dtype == 0 ? 15 : 7;
+    return V % 4 == 0 && ld_base % 4 == 0 && (reinterpret_cast<uintptr_t>(base) & align) == 0;
 }
 
 }  // namespace dels

@@ -20,11 +20,10 @@
 //   * rank: workgroups 0 .. r/16 - 1 each own one 16-column tile of the rank
 //     and keep its 16 rows of A in LDS; rank = bf16(act(bf16(h . A^T + b)))
 //     goes out as words {tag, two bf16}, read by every workgroup;
-//   * argmax: every wave contracts its resident tiles against the rank
-//     (v_mfma_f32_16x16x32_bf16, lane l holding rows 4(l/16)+q of column
-//     l%16), combines s = fma(-beta, prior, fma(dot, alpha, base)) as every
-//     kernel of the path does, and keeps a running (score, index) per lane;
-//     the workgroup publishes each row's best as one slot word (order(score)
+//   * argmax: every wave contracts its resident tiles against the rank and
+//     combines s = fma(-beta, prior, fma(dot, alpha, base)) as every kernel of
+//     the path does (rr_tiles_best: 2.2 us of an 11.1 us step with a running
+//     (score, index) pair for each of a lane's four rows, 1.65 here; 8 rows); the workgroup publishes each row's best as one slot word (order(score)
 //     in the high half, ~index above two flag bits in the low half, so the
 //     larger word is the argmax with ties to the lower index) and every
 //     workgroup reads all nwg slots of each row, takes the maximum and so
@@ -49,7 +48,7 @@
 // Up to 16 rows run as one group.  17 to 32 run as two (see the kernel); a launch
 // that cannot finish them leaves the rollout to the ordered one behind it.  14
 // steps of 24 rows at V = 151936, G = 1024, with the copies of a runner's call:
-// 577.9 us as per-step launches (argmax 17 us, GRU 8.6, rank 7.7 a step), 307.9 here.
+// 577.9 us as per-step launches (argmax 17 us, GRU 8.6, rank 7.7 a step), 295.3 here.
 #include <algorithm>
 #include <climits>
 
@@ -94,7 +93,7 @@ struct RrArgs {
 // workgroup reads more state words than with 16 rows; every workgroup contracts
 // its tiles of B with both groups' ranks.  A group's rows are numbered from its
 // first: M rows of the group from row m0 of the batch.
-template <int RG, typename BaseT, typename PriorT>
+template <int RG, typename BaseT, typename PriorT, bool VEC>
 __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) {
 #pragma clang fp contract(off)
     constexpr int kUnitTiles = RG;                  // operand tiles of W_hh rows: RG * 4 units x 3 gates
@@ -104,7 +103,7 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     __shared__ __attribute__((aligned(16))) char s_union[kRrUnionBytes];       // A rows (rank WGs) or B tiles
     __shared__ __attribute__((aligned(16))) uint16_t s_rank[RG * 16 * kRrRPitch];
     __shared__ __attribute__((aligned(16))) float s_red[RG * kRrWaves * 256];
-    __shared__ float s_prior[(kRrWaves * kRrRegTiles + kResidentLdsTiles) * 16];
+    __shared__ __attribute__((aligned(16))) float s_prior[kRrPriorWords];
     __shared__ unsigned long long s_key[kRrWaves][RG * 16];    // each wave's best key of each row
     __shared__ float s_gh[16 * kGhPitch];
     __shared__ float s_ab[2][kResidentMaxSteps];          // alpha, beta of each step
@@ -380,6 +379,7 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         *reinterpret_cast<u32x4*>(s_whh + kb * 1024 + l * 16) = v;
     }
     // the prior of every column of the workgroup's tiles (widened)
+    if (threadIdx.x < 16) s_prior[kRrPriorZeros + threadIdx.x] = 0.f;
     for (int i = threadIdx.x; i < ntl * 16; i += kRrThreads) {
         const int v = min(T0 * 16 + i, V - 1);
         if constexpr (is_no_prior<PriorT>::value) s_prior[i] = 0.f;
@@ -421,22 +421,14 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         int lcol = col, lkg = kg;
         asm volatile("" : "+v"(lcol), "+v"(lkg));
         if (rank_wg) rank_publish(tag);
-        // base values of this wave's tiles (issued before the rank wait): the
-        // wave-uniform start of each tile's columns plus one per-lane offset per row
-        uint32_t braw[kRrRegTiles + 1][4];
+        // base values of this wave's tiles, issued before the rank wait; the second
+        // group's after it where they are two words a tile, else when its turn comes
+        constexpr bool kBoth = RG == 2 && sizeof(BaseT) == 2;
+        RrBase<BaseT> braw[kBoth ? 2 : 1];
         auto load_base = [&](int g) __attribute__((always_inline)) {
-            const BaseT* bs = base + (int64_t)s * V;
-#pragma unroll
-            for (int j = 0; j <= kRrRegTiles; ++j) {
-                const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
-                const int tc = min(T0 + min(ti, max(ntl - 1, 0)), a.ntiles - 1);
-                const int vc = min(tc * 16 + lcol, V - 1);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int m = 16 * g + 4 * lkg + q;
-                    braw[j][q] = load_raw(bs + (int64_t)(m < a.M ? m : 0) * a.ld_base + vc);
-                }
-            }
+            const int m = 16 * g + lcol;
+            rr_load_base<BaseT, VEC>(base + (int64_t)s * V + (int64_t)(m < a.M ? m : 0) * a.ld_base, T0, ntl,
+                                     a.ntiles, wave, lkg, V, braw[kBoth ? g : 0]);
         };
         load_base(0);
         // keep these loads ahead of the rank wait (the compiler would otherwise
@@ -444,72 +436,18 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         asm volatile("" ::: "memory");
         ok = read_rank(tag);
         if (!ok) break;
+        if constexpr (kBoth) load_base(1);
 
         // ---- argmax over the resident tiles -------------------------------------
-        // K step outermost: each rank operand is read from LDS once and feeds
-        // every tile's accumulator
-        const float al = s_ab[0][s], be = s_ab[1][s];
-        const bool use_prior = !is_no_prior<PriorT>::value && be != 0.f;
         const bool lds_tile = !rank_wg && has_lds_tile;
+        const char* ltile = s_union + (lds_tile ? wave : 0) * kRrKs * 1024;
 #pragma unroll
         for (int g = 0; g < RG; ++g) {
-            if (g > 0) load_base(g);
-            f32x4 acc[kRrRegTiles + 1];
-#pragma unroll
-            for (int j = 0; j <= kRrRegTiles; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-            // unconditional contractions (no branches between the MFMAs): a tile that
-            // is not this wave's holds zeros, or for the LDS slot of a wave without
-            // one any data, and is not combined
-            const int lslot = lds_tile ? wave : 0;
-#pragma unroll
-            for (int k = 0; k < kRrKs; ++k) {
-                const bf16x8 rk = *reinterpret_cast<const bf16x8*>(&s_rank[(16 * g + lcol) * kRrRPitch + k * 32 + lkg * 8]);
-                const bf16x8 bv = *reinterpret_cast<const bf16x8*>(s_union + (lslot * kRrKs + k) * 1024 + lane * 16);
-#pragma unroll
-                for (int j = 0; j < kRrRegTiles; ++j)
-                    acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bt[j][k], acc[j], 0, 0, 0);
-                acc[kRrRegTiles] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rk, bv, acc[kRrRegTiles], 0, 0, 0);
-            }
-            float best[4];
-            int bidx[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) { best[q] = -__builtin_inff(); bidx[q] = INT_MAX; }
-            // a lane's column grows with its tile number, so a later tile takes the
-            // lead only on a larger score, or on an equal one while nothing has
-            // (the first -inf); written with bitwise tests, no branches
-#pragma unroll
-            for (int j = 0; j <= kRrRegTiles; ++j) {
-                const int ti = j < kRrRegTiles ? wave + 8 * j : kRrWaves * kRrRegTiles + wave;
-                const bool live = j < kRrRegTiles ? ti < ntl : lds_tile;   // wave-uniform
-                const int tc = min(ti, max(ntl - 1, 0));
-                const int v = (T0 + tc) * 16 + lcol;
-                const bool livev = live & (v < V);
-                const float pv = s_prior[tc * 16 + lcol];
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    float sc = __builtin_fmaf(acc[j][q], al, widen_raw<BaseT>(braw[j][q]));
-                    if (use_prior) sc = __builtin_fmaf(-be, pv, sc);
-                    const bool take = livev & ((sc > best[q]) | ((sc == best[q]) & (bidx[q] == INT_MAX)));
-                    best[q] = take ? sc : best[q];
-                    bidx[q] = take ? v : bidx[q];
-                }
-            }
-            // over the 16 columns of each row as argmax keys (a lane without a
-            // candidate holds -inf at index INT_MAX, below every real one; DPP row
-            // shifts: lane 15 of a row ends with the row's best), then (below) the waves
-            unsigned long long key[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                key[q] = pack_argmax(best[q], (uint32_t)bidx[q]);
-                rr_row_max<1>(key[q]);
-                rr_row_max<2>(key[q]);
-                rr_row_max<4>(key[q]);
-                rr_row_max<8>(key[q]);
-            }
-            if (col == 15) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) s_key[wave][16 * g + 4 * kg + q] = key[q];
-            }
+            if (g > 0 && !kBoth) load_base(g);
+            const unsigned long long key = rr_tiles_best<kRrKs, true, BaseT, PriorT, VEC>(
+                bt, ltile, lds_tile, &s_rank[(16 * g + lcol) * kRrRPitch + lkg * 8], braw[kBoth ? g : 0], s_prior, T0,
+                ntl, wave, lkg, V, s_ab[0][s], s_ab[1][s]);
+            if (kg == 0) s_key[wave][16 * g + col] = key;
         }
         __syncthreads();
         // the workgroup's best of each row into its slot word for the step
@@ -600,23 +538,27 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
     }
 }
 
-template <int RG, typename BaseT>
+template <int RG, typename BaseT, bool VEC>
 hipError_t launch_rr_base(const RrArgs& a, int prior_kind, int nwg, hipStream_t s) {
     const dim3 grid(nwg), block(kRrThreads);
     switch (prior_kind) {
-        case 0: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, no_prior_t>), grid, block, 0, s, a); break;
-        case 1: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, float>), grid, block, 0, s, a); break;
-        case 2: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, bf16_t>), grid, block, 0, s, a); break;
-        default: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, f16_t>), grid, block, 0, s, a); break;
+        case 0: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, no_prior_t, VEC>), grid, block, 0, s, a); break;
+        case 1: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, float, VEC>), grid, block, 0, s, a); break;
+        case 2: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, bf16_t, VEC>), grid, block, 0, s, a); break;
+        default: hipLaunchKernelGGL((rollout_resident_kernel<RG, BaseT, f16_t, VEC>), grid, block, 0, s, a); break;
     }
     return hipGetLastError();
 }
 
 template <int RG>
 hipError_t launch_rr(const RrArgs& a, int base_dtype, int prior_kind, int nwg, hipStream_t s) {
-    if (base_dtype == 1) return launch_rr_base<RG, bf16_t>(a, prior_kind, nwg, s);
-    if (base_dtype == 2) return launch_rr_base<RG, f16_t>(a, prior_kind, nwg, s);
-    return launch_rr_base<RG, float>(a, prior_kind, nwg, s);
+    auto by_base = [&](auto vec) -> hipError_t {
+        constexpr bool VEC = decltype(vec)::value;
+        if (base_dtype == 1) return launch_rr_base<RG, bf16_t, VEC>(a, prior_kind, nwg, s);
+        if (base_dtype == 2) return launch_rr_base<RG, f16_t, VEC>(a, prior_kind, nwg, s);
+        return launch_rr_base<RG, float, VEC>(a, prior_kind, nwg, s);
+    };
+    return rr_vec(a.base, base_dtype, a.ld_base, a.V) ? by_base(std::true_type{}) : by_base(std::false_type{});
 }
 
 int g_resident_spin_limit = 1 << 16;   // re-reads before a wait gives up (each ~1-2 us)
