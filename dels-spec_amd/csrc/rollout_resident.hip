@@ -502,6 +502,11 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         }
         if (s + 1 < a.steps) {
             gru_publish(s_ids, 1, rr_tag(gen, s + 1));
+            // the other workgroups read the state later than those that project the
+            // rank from it: 8 MB of words (8 rows) on their way to everyone at once
+            // delay the ones that the step waits for (8 rows 10.45 -> 10.1 us a step,
+            // 24 rows 17.0 -> 16.2; half the pause gains nothing, more loses again)
+            if (!rank_wg) __builtin_amdgcn_s_sleep(RG == 1 ? 40 : 56);
             ok = read_state(rr_tag(gen, s + 1));
         }
     }
