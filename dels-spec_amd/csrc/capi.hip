@@ -813,6 +813,10 @@ int dels_fused_argmax(const void* rank, int64_t ldrank, const void* B, int64_t l
 int dels_debug_set_decode_spin_limit(int limit) { return set_decode_spin_limit(limit); }
 int dels_debug_set_rollout_resident(int enable) { return set_rollout_resident(enable); }
 int dels_debug_set_resident_spin_limit(int limit) { return set_resident_spin_limit(limit); }
+int dels_debug_set_ordered_wait_limit(int limit) {
+    set_ordered_wait_limit(limit);
+    return DELS_OK;
+}
 
 size_t dels_lowrank_argmax_ws_bytes(int64_t M, int64_t d, int64_t r, int64_t V) {
     if (!rows_ok(M) || !inner_ok(d) || !rows_ok(r) || !vocab_ok(V)) return 0;

@@ -217,6 +217,7 @@ hipError_t launch_rollout_resident(const ResidentRolloutArgs& a, void* ws, hipSt
 hipError_t launch_rollout_ordered(const ResidentRolloutArgs& a, void* ws, hipStream_t s);
 int resident_spin_limit();
 int set_resident_spin_limit(int limit);   // returns the previous limit
+void set_ordered_wait_limit(int limit);   // < 0: the default
 int set_rollout_resident(int enable);   // returns the previous setting (1 = used where eligible)
 bool rollout_resident_enabled();
 // The Markov rollout with B resident on chip (markov_resident.hip: r = 128 or

@@ -11,8 +11,11 @@
 // kOrdChunks argmax tasks over chunks of the vocabulary; a task waits for every
 // task of the phase before its own.  Those have lower tickets, so they are held
 // by workgroups that are already running and themselves only wait for lower
-// tickets: every wait ends, however few workgroups run at a time.  Correctness
-// is the point, not speed: B streams through the caches every step (as in the
+// tickets: every wait ends, however few workgroups run at a time.  All the same
+// each is bounded (a control area that was not clean could leave a count short
+// for ever): one that runs out reports it in the error word, the workgroups stop
+// taking tasks, and the last one writes ids of -1 and leaves the control area
+// clean.  Correctness is the point, not speed: B streams through the caches every step (as in the
 // per-step launches), and what another workgroup wrote is read with
 // device-scope loads.  Sums run in the resident kernels' order, so the results
 // are theirs bit for bit.
@@ -40,6 +43,7 @@ struct OrderedArgs {
     int64_t* out_ids; float* out_scores; int64_t ld_out;
     unsigned int* counters;
     unsigned long long* keys;                                 // [steps][32]
+    int wait_limit;                                           // looks at a phase's count before giving up
 };
 
 // Table row of row m's token at step s: given for step 0, else the index in its key of step s - 1.
@@ -226,6 +230,17 @@ __device__ __forceinline__ void ordered_argmax(const OrderedArgs& a, int s, int 
     asm volatile("" ::"v"(seen));   // the maxima have returned
 }
 
+// Wait until a phase's count of finished tasks reaches `want`.  False when it did
+// not within wait_limit looks, or another workgroup gave up.
+__device__ __forceinline__ bool ordered_wait(const OrderedArgs& a, const unsigned int* count, unsigned want) {
+    for (int it = 0; it < a.wait_limit; ++it) {
+        if (__hip_atomic_load(count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want) return true;
+        if ((it & 63) == 63 && rr_failed(a)) return false;
+        __builtin_amdgcn_s_sleep(8);
+    }
+    return false;
+}
+
 template <bool GRU, int KS, typename BaseT, typename PriorT>
 __global__ __launch_bounds__(kRrThreads) void rollout_ordered_kernel(OrderedArgs a) {
     __shared__ unsigned long long s_key[kRrWaves][32];
@@ -241,8 +256,8 @@ __global__ __launch_bounds__(kRrThreads) void rollout_ordered_kernel(OrderedArgs
     for (;;) {
         __syncthreads();   // the LDS of the task before has been read
         if (threadIdx.x == 0) {
-            const unsigned t = __hip_atomic_fetch_add(a.counters + kRrTicketWord, 1u, __ATOMIC_RELAXED,
-                                                      __HIP_MEMORY_SCOPE_AGENT);
+            unsigned t = __hip_atomic_fetch_add(a.counters + kRrTicketWord, 1u, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
             if (t < total) {
                 // the phase before this task's: its counter and how many tasks it has
                 const unsigned s = t / per, i = t % per;
@@ -251,9 +266,10 @@ __global__ __launch_bounds__(kRrThreads) void rollout_ordered_kernel(OrderedArgs
                 unsigned want = 0;
                 if (GRU && ph > 0) { before = done + s * 3 + ph - 1; want = ph == 1 ? n0 : n1; }
                 else if (s > 0) { before = done + (s - 1) * 3 + 2; want = kOrdChunks; }
-                if (before)
-                    while (__hip_atomic_load(before, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != want)
-                        __builtin_amdgcn_s_sleep(8);
+                if (before && !ordered_wait(a, before, want)) {
+                    rr_fail(a);
+                    t = total;
+                }
             }
             s_task = t;
         }
@@ -278,28 +294,35 @@ __global__ __launch_bounds__(kRrThreads) void rollout_ordered_kernel(OrderedArgs
             __hip_atomic_fetch_add(done + s * 3 + ph, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     // the last workgroup to run out of tasks decodes the keys and leaves the control area clean
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_s_waitcnt(0);   // a failure is stored before this workgroup counts as out of tasks
         s_task = __hip_atomic_fetch_add(a.counters + kRrExitCounter, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __syncthreads();
     if (s_task != gridDim.x - 1) return;
+    const bool failed = rr_failed(a);
+    __syncthreads();   // every thread has read the error word before it is cleared
     for (int i = threadIdx.x; i < a.steps * 32; i += kRrThreads) {
         const int s = i >> 5, m = i & 31;
         const unsigned long long k = __hip_atomic_exchange(a.keys + i, 0ull, __ATOMIC_RELAXED,
                                                            __HIP_MEMORY_SCOPE_AGENT);
         if (m >= a.M) continue;
-        uint32_t idx = ~(uint32_t)k;
+        int64_t id = (int64_t)(uint32_t)~(uint32_t)k;
         float val = f32_from_order_key((uint32_t)(k >> 32));
-        if (k == 0ull || idx >= (uint32_t)a.V) {   // no candidate at all
-            idx = 0;
+        if (failed || k == 0ull || id >= a.V) {    // not produced, or no candidate at all
+            id = failed ? -1 : 0;
             val = -__builtin_inff();
         }
-        a.out_ids[(int64_t)m * a.ld_out + s] = (int64_t)idx;
+        a.out_ids[(int64_t)m * a.ld_out + s] = id;
         if (a.out_scores) a.out_scores[(int64_t)m * a.ld_out + s] = val;
     }
     for (int i = threadIdx.x; i < a.steps * 3; i += kRrThreads)
         __hip_atomic_store(done + i, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (threadIdx.x < 3) {
-        const int word = threadIdx.x == 0 ? kRrNotDoneWord : threadIdx.x == 1 ? kRrTicketWord : kRrExitCounter;
+    if (threadIdx.x < 4) {
+        const int word = threadIdx.x == 0   ? kRrNotDoneWord
+                         : threadIdx.x == 1 ? kRrTicketWord
+                         : threadIdx.x == 2 ? kRrExitCounter
+                                            : kRrErrorWord;
         __hip_atomic_store(a.counters + word, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
@@ -324,7 +347,12 @@ hipError_t launch_ordered_base(const OrderedArgs& a, const void* prior, int prio
     return launch_ordered<GRU, KS, float>(a, pk, s);
 }
 
+constexpr int kOrdWaitLimit = 1 << 22;   // looks (about 1 us each) before a wait gives up
+int g_ordered_wait_limit = kOrdWaitLimit;
+
 }  // namespace
+
+void set_ordered_wait_limit(int limit) { g_ordered_wait_limit = limit < 0 ? kOrdWaitLimit : limit; }
 
 hipError_t launch_markov_ordered(const MarkovRolloutArgs& r, hipStream_t s) {
     OrderedArgs a{};
@@ -338,6 +366,7 @@ hipError_t launch_markov_ordered(const MarkovRolloutArgs& r, hipStream_t s) {
     a.out_ids = r.out_ids; a.out_scores = r.out_scores; a.ld_out = r.ld_out;
     a.counters = r.counters;
     a.keys = r.keys;
+    a.wait_limit = g_ordered_wait_limit;
     if (r.r == 256) return launch_ordered_base<false, 8>(a, r.prior, r.prior_dtype, r.base_dtype, s);
     return launch_ordered_base<false, 4>(a, r.prior, r.prior_dtype, r.base_dtype, s);
 }
@@ -358,6 +387,7 @@ hipError_t launch_rollout_ordered(const ResidentRolloutArgs& r, void* ws, hipStr
     a.out_ids = r.out_ids; a.out_scores = r.out_scores; a.ld_out = r.ld_out;
     a.counters = reinterpret_cast<unsigned int*>(w + kCountersOff);
     a.keys = reinterpret_cast<unsigned long long*>(w + kKeysOff);
+    a.wait_limit = g_ordered_wait_limit;
     return launch_ordered_base<true, kResidentRank / 32>(a, r.prior, r.prior_dtype, r.base_dtype, s);
 }
 

@@ -233,6 +233,12 @@ int dels_debug_set_rollout_resident(int enable);
  * rollout, and more than 16 rows: leaves the whole rollout to the launch that
  * follows it), and the next launch starts clean.  Returns the previous limit.  Not thread-safe. */
 int dels_debug_set_resident_spin_limit(int limit);
+/* Test hook: the launch that follows a Markov rollout, or one of more than 16
+ * rows, and does it when the one-launch rollout gave up, looks at most `limit`
+ * times at the count that a piece of its work waits for (0: gives up at the first
+ * wait; < 0: the default, 2^22); then the rollout's ids are all -1, its scores
+ * -inf, and the next launch starts clean.  Returns DELS_OK.  Not thread-safe. */
+int dels_debug_set_ordered_wait_limit(int limit);
 
 /*
  * Plain argmax of each row of logits: sample() at temperature 0
