@@ -211,7 +211,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(Argma
                     tr.b[s], *reinterpret_cast<const bf16x8*>(s_rank + (s * RG + g) * 1024 + lo), acc[g], 0, 0, 0);
         const int v = t * 16 + 4 * kg;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 3; q >= 0; --q) {
             const bool in = v + q < a.V;
             float pv = 0.f;
             if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
@@ -219,38 +219,41 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(Argma
             for (int g = 0; g < RG; ++g) {
                 float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT, VEC>(tr.base[g], q));
                 if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
-                // a lane's candidates arrive in increasing column order: strict ">" keeps the lowest index
-                const bool take = in & (sc > best[g]);
+                // a lane's candidates arrive in decreasing column order: ">=" ends at the lowest index,
+                // that of a first score of -inf among them
+                const bool take = in & (sc >= best[g]);
                 best[g] = take ? sc : best[g];
                 bidx[g] = take ? v + q : bidx[g];
             }
         }
     };
 
-    // the tiles t + k * nwaves, k < cnt, through two register sets (see the GEMV kernel)
+    // the wave's tiles t, t + nwaves, .. (cnt of them), the last one first, through two
+    // register sets (see the GEMV kernel)
     const int ntiles = (a.V + 15) >> 4;
     const int nwaves = gridDim.x * kWaves;
     const int t = blockIdx.x * kWaves + wave;
     const int cnt = t < ntiles ? (ntiles - 1 - t) / nwaves + 1 : 0;
+    const int te = t + (cnt - 1) * nwaves;
     Tile tr0, tr1;
     // the first two whether or not the wave has them, so that the waits below are exact
-    load(cnt > 0 ? t : 0, cnt > 0, tr0);
-    load(cnt > 1 ? t + nwaves : 0, cnt > 1, tr1);
+    load(cnt > 0 ? te : 0, cnt > 0, tr0);
+    load(cnt > 1 ? te - nwaves : 0, cnt > 1, tr1);
 #pragma unroll
     for (int i = 0; i < kPieces; ++i)
         *reinterpret_cast<u32x4*>(s_rank + (threadIdx.x + kThreads * i) * 16) = rp[i];
     lds_barrier();   // the stream's loads stay in flight
     int k = 0;
     for (; k + 4 <= cnt; k += 2) {
-        consume(tr0, t + k * nwaves);
-        load(t + (k + 2) * nwaves, true, tr0);
-        consume(tr1, t + (k + 1) * nwaves);
-        load(t + (k + 3) * nwaves, true, tr1);
+        consume(tr0, te - k * nwaves);
+        load(te - (k + 2) * nwaves, true, tr0);
+        consume(tr1, te - (k + 1) * nwaves);
+        load(te - (k + 3) * nwaves, true, tr1);
     }
-    if (k < cnt) consume(tr0, t + k * nwaves);
-    if (k + 2 < cnt) load(t + (k + 2) * nwaves, true, tr0);
-    if (k + 1 < cnt) consume(tr1, t + (k + 1) * nwaves);
-    if (k + 2 < cnt) consume(tr0, t + (k + 2) * nwaves);
+    if (k < cnt) consume(tr0, te - k * nwaves);
+    if (k + 2 < cnt) load(te - (k + 2) * nwaves, true, tr0);
+    if (k + 1 < cnt) consume(tr1, te - (k + 1) * nwaves);
+    if (k + 2 < cnt) consume(tr0, te - (k + 2) * nwaves);
 
     rows_finish<RG>(a, best, bidx, m0, s_val, s_idx, s_last);
 }

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
             }
         const int v = t * 16 + 4 * kg;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 3; q >= 0; --q) {
             const bool in = v + q < a.V;
             const float bs = __uint_as_float(tr.bscale[q]);
             float pv = 0.f;
@@ -130,23 +130,26 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
                 dot = dot * bs;
                 float sc = __builtin_fmaf(dot, al[g], quad_at<BaseT, VEC>(tr.base[g], q));
                 if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
-                // a lane's candidates arrive in increasing column order: strict ">" keeps the lowest index
-                const bool take = in & (sc > best[g]);
+                // a lane's candidates arrive in decreasing column order: ">=" ends at the lowest index,
+                // that of a first score of -inf among them
+                const bool take = in & (sc >= best[g]);
                 best[g] = take ? sc : best[g];
                 bidx[g] = take ? v + q : bidx[g];
             }
         }
     };
 
-    // the tiles t + k * nwaves, k < cnt, through kND register sets (see the GEMV kernel)
+    // the wave's tiles t, t + nwaves, .. (cnt of them), the last one first, through kND
+    // register sets (see the GEMV kernel)
     const int ntiles = (a.V + 15) >> 4;
     const int nwaves = gridDim.x * kWaves;
     const int t = blockIdx.x * kWaves + wave;
     const int cnt = t < ntiles ? (ntiles - 1 - t) / nwaves + 1 : 0;
+    const int te = t + (cnt - 1) * nwaves;
     Tile tr[kND];
     // the first ones whether or not the wave has them, so that the waits below are exact
 #pragma unroll
-    for (int u = 0; u < kND; ++u) load(u < cnt ? t + u * nwaves : 0, u < cnt, tr[u]);
+    for (int u = 0; u < kND; ++u) load(u < cnt ? te - u * nwaves : 0, u < cnt, tr[u]);
 
     // the rank rows, quantised by the rule of quantize_rank_coop, into operand
     // order: a thread's bytes are whole 16-byte pieces of one K128 block
@@ -187,18 +190,18 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
     for (; k + 2 * kND <= cnt; k += kND) {
 #pragma unroll
         for (int u = 0; u < kND; ++u) {
-            consume(tr[u], t + (k + u) * nwaves);
-            load(t + (k + u + kND) * nwaves, true, tr[u]);
+            consume(tr[u], te - (k + u) * nwaves);
+            load(te - (k + u + kND) * nwaves, true, tr[u]);
         }
     }
 #pragma unroll
     for (int u = 0; u < kND; ++u) {
-        if (k + u < cnt) consume(tr[u], t + (k + u) * nwaves);
-        if (k + u + kND < cnt) load(t + (k + u + kND) * nwaves, true, tr[u]);
+        if (k + u < cnt) consume(tr[u], te - (k + u) * nwaves);
+        if (k + u + kND < cnt) load(te - (k + u + kND) * nwaves, true, tr[u]);
     }
 #pragma unroll
     for (int u = 0; u < kND; ++u)
-        if (k + u + kND < cnt) consume(tr[u], t + (k + u + kND) * nwaves);
+        if (k + u + kND < cnt) consume(tr[u], te - (k + u + kND) * nwaves);
 
     rows_finish<RG>(a, best, bidx, m0, s_val, s_idx, s_last);
 }
