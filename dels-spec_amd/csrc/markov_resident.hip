@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
         const char* ltile = s_b + (lds_tile ? wave : 0) * KS * 1024;
 #pragma unroll
         for (int g = 0; g < RG; ++g) {
-            const unsigned long long key = rr_tiles_best<KS, false, BaseT, PriorT, VEC>(
+            const unsigned long long key = rr_tiles_best<KS, BaseT, PriorT, VEC>(
                 bt, ltile, lds_tile, &s_rank[(16 * g + lcol) * kPitch + lkg * 8], braw[g], s_prior, T0, ntl, wave, lkg,
                 V, s_ab[0][s], s_ab[1][s]);
             if (kg == 0) s_key[wave][16 * g + col] = key;

@@ -202,7 +202,7 @@ __device__ __forceinline__ void ordered_argmax(const OrderedArgs& a, int s, int 
             for (int q = 0; q < 4; ++q) {
                 float sc = __builtin_fmaf(acc[q], al, load_f32(brow[q] + vc));
                 if (use_prior) sc = __builtin_fmaf(-be, pv, sc);
-                const bool take = (v < a.V) & (sc > best[q]);
+                const bool take = (v < a.V) & argmax_better(sc, v, best[q], bidx[q]);
                 best[q] = take ? sc : best[q];
                 bidx[q] = take ? v : bidx[q];
             }

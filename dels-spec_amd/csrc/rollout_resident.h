@@ -263,8 +263,8 @@ __device__ __forceinline__ void rr_shift_quad(RrQuad<BaseT>& w, int v, int V) {
 // column: twenty 2-byte loads, four pairs and sixteen exchanges.)  K step
 // outermost: each rank operand is read from LDS once and feeds every tile; no
 // branches between the MFMAs: a tile that is not the wave's is not combined.
-// TAKE_INF: a row whose best score is -inf names its first column at that score.
-template <int KS, bool TAKE_INF, typename BaseT, typename PriorT, bool VEC>
+// A row whose best score is -inf names its first column at that score.
+template <int KS, typename BaseT, typename PriorT, bool VEC>
 __device__ __forceinline__ unsigned long long rr_tiles_best(const bf16x8 (&bt)[kRrRegTiles][KS], const char* ltile,
                                                             bool lds_tile, const uint16_t* rank,
                                                             RrBase<BaseT>& braw, const float* s_prior,
@@ -314,8 +314,7 @@ __device__ __forceinline__ unsigned long long rr_tiles_best(const bf16x8 (&bt)[k
     int cand = -1;
 #pragma unroll
     for (int c = 4 * kRrRegTiles + 3; c >= 0; --c) cand = acc[c >> 2][c & 3] == best ? c : cand;
-    if constexpr (!TAKE_INF) cand = best == -__builtin_inff() ? -1 : cand;
-    // candidate 4 j + q is column (T0 + wave + 8 j) * 16 + 4 kg + q; none: INT_MAX
+    // candidate 4 j + q is column (T0 + wave + 8 j) * 16 + 4 kg + q; none (every score NaN): INT_MAX
     const int idx = cand < 0 ? INT_MAX : (T0 + wave + 8 * (cand >> 2)) * 16 + 4 * kg + (cand & 3);
     unsigned long long key = pack_argmax(best, (uint32_t)idx);
 #pragma unroll

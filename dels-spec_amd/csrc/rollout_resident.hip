@@ -444,7 +444,7 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
 #pragma unroll
         for (int g = 0; g < RG; ++g) {
             if (g > 0 && !kBoth) load_base(g);
-            const unsigned long long key = rr_tiles_best<kRrKs, true, BaseT, PriorT, VEC>(
+            const unsigned long long key = rr_tiles_best<kRrKs, BaseT, PriorT, VEC>(
                 bt, ltile, lds_tile, &s_rank[(16 * g + lcol) * kRrRPitch + lkg * 8], braw[kBoth ? g : 0], s_prior, T0,
                 ntl, wave, lkg, V, s_ab[0][s], s_ab[1][s]);
             if (kg == 0) s_key[wave][16 * g + col] = key;
