@@ -167,7 +167,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
             uint32_t low = 0u;
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const float y = __builtin_fminf(xv[q] * s_a, xv[q] * s_b);
+                float y = __builtin_fminf(xv[q] * s_a, xv[q] * s_b);
+                // a float16 quotient may round to -inf (as for y_upper)
+                if constexpr (std::is_same<T, f16_t>::value) y = y < -65000.f ? -__builtin_inff() : y;
                 const float lo = __builtin_fmaf(__builtin_amdgcn_logf((float)(c[q] >> 9) + 0.5f) - lu[q], kLn2,
                                                 y - kBoundSlack);
                 const bool use = (xv[q] == xv[q]) & (lo == lo) & (VEC || g + q < v1);
@@ -185,7 +187,9 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
             if (!(up[q] <= thr)) {
                 const float val = tempered(xv[q], temperature, T{}) + gumbel_from_bits(c[q]);
                 const unsigned long long k = sample_key(val, (uint32_t)(g + q));
-                best = k > best ? k : best;
+                // -inf is no candidate: not every such element is evaluated, and a row of
+                // nothing else gives id 0 without one
+                best = val != -__builtin_inff() && k > best ? k : best;
                 if (val == val) atomicMax(&s_thr, f32_order_key(val));
             }
         }

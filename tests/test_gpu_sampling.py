@@ -141,3 +141,29 @@ def test_sample_rows_skipped_candidates_change_nothing(pkg, dev, dtype, V, pad):
     assert ids[2] == 0 and score[2] == -np.inf
     assert ids[5] == V // 3 and score[5] == np.inf
     assert ids[6] == V // 2 and np.isnan(score[6])
+
+
+@pytest.mark.parametrize("V", [3, 1023, 4096, 30005])
+def test_sample_rows_float16_quotients_past_the_range(pkg, dev, V):
+    """float16 logits whose quotients round to -inf take no part, and neither hide nor precede those
+    that stay finite: a row of only such quotients gives id 0 at -inf, as a masked row does."""
+    print(f"case sampling float16 range V={V}", flush=True)
+    T, seed = 0.7, 11
+    x = torch.full((6, V), -65504.0, dtype=torch.float16)         # / 0.7: -inf
+    x[1, 0] = float("-inf")
+    x[2] = float("-inf")
+    x[2, V // 2] = -65504.0
+    x[3, V - 1] = -40000.0                                        # the only finite quotient
+    x[4] = -45872.0                                               # / 0.7 = -65531: past the range, by less than noise
+    x[4, V // 3] = -45824.0                                       # / 0.7 = -65463: the only finite one
+    g = torch.Generator().manual_seed(V)
+    x[5] = (torch.randn(V, generator=g) * 30000.0).clamp(-65504.0, 65504.0).to(torch.float16)
+    ids, score = pkg.sample_rows(x.to(dev), T, seed)
+    torch.cuda.synchronize()
+    s = S.perturbed_scores(x.float().numpy(), T, seed, 0, "float16")
+    assert np.isinf(s[:3]).all() and np.isfinite(s[3]).sum() == 1 and np.isfinite(s[4]).sum() == 1
+    ids, score = ids.cpu().numpy(), score.cpu().numpy()
+    assert list(ids[:5]) == [0, 0, 0, V - 1, V // 3]
+    assert np.all(score[:3] == -np.inf) and np.all(np.isfinite(score[3:5]))
+    best = s[5].max()
+    assert s[5, ids[5]] == best if np.isinf(best) else s[5, ids[5]] >= best - 1e-5 * max(1.0, abs(best))
