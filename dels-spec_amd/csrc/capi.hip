@@ -751,8 +751,8 @@ int dels_pack_operand(const void* W, int64_t ldw, int64_t rows, int64_t cols, vo
 
 size_t dels_rank_proj_ws_bytes(int64_t M, int64_t d, int64_t r) {
     if (!rows_ok(M) || !inner_ok(d) || !rows_ok(r)) return 0;
-    return kDataOff + skinny_data_bytes(plan_skinny(std::max<int64_t>(M, 1), std::max<int64_t>(d, 1),
-                                                      std::max<int64_t>(r, 1), false));
+    return kDataOff + skinny_data_bytes_upto(std::max<int64_t>(M, 1), std::max<int64_t>(d, 1),
+                                             std::max<int64_t>(r, 1), false);
 }
 
 int dels_rank_proj(const void* h, int64_t ldh, const void* A, int64_t lda, int a_layout, const void* bias, int act,
@@ -820,8 +820,9 @@ int dels_debug_set_ordered_wait_limit(int limit) {
 
 size_t dels_lowrank_argmax_ws_bytes(int64_t M, int64_t d, int64_t r, int64_t V) {
     if (!rows_ok(M) || !inner_ok(d) || !rows_ok(r) || !vocab_ok(V)) return 0;
-    return lowrank_layout(std::max<int64_t>(M, 1), std::max<int64_t>(d, 1), std::max<int64_t>(r, 1),
-                          std::max<int64_t>(V, 1)).total;
+    M = std::max<int64_t>(M, 1), d = std::max<int64_t>(d, 1), r = std::max<int64_t>(r, 1), V = std::max<int64_t>(V, 1);
+    const LowrankLayout L = lowrank_layout(M, d, r, V);
+    return L.total - skinny_data_bytes(L.plan) + skinny_data_bytes_upto(M, d, r, false);
 }
 
 int dels_lowrank_argmax(const void* h, int64_t ldh, const void* A, int64_t lda, int a_layout, const void* bias,
@@ -881,7 +882,10 @@ int dels_lowrank_argmax_noalloc(const void* h, int64_t ldh, const void* A, int64
                                 int prior_dtype, const float* alpha, int64_t alpha_stride, const float* beta,
                                 int64_t beta_stride, int64_t M, int64_t d, int64_t r, int64_t V, int64_t* out_ids,
                                 float* out_score, int64_t ld_out, void* stream) {
-    const size_t need = dels_lowrank_argmax_ws_bytes(M, d, r, V);
+    // what this call takes (shapes past the extents: 0, refused below)
+    const size_t need = rows_ok(M) && inner_ok(d) && rows_ok(r) && vocab_ok(V) && M > 0 && d > 0 && r > 0 && V > 0
+                            ? lowrank_layout(M, d, r, V).total
+                            : 0;
     if (need > DELS_NOALLOC_SCRATCH_BYTES)
         return fail(DELS_ERR_WORKSPACE,
                     "dels_lowrank_argmax_noalloc: M=%lld d=%lld r=%lld V=%lld needs %zu bytes of scratch, more "
@@ -1087,8 +1091,8 @@ int dels_sample_rows(const void* x, int64_t ldx, int dtype, int64_t M, int64_t V
 
 size_t dels_gru_step_ws_bytes(int64_t batch, int64_t G) {
     if (!rows_ok(batch) || !rows_ok(G)) return 0;
-    return kDataOff + skinny_data_bytes(plan_skinny(std::max<int64_t>(batch, 1), std::max<int64_t>(G, 1),
-                                                      std::max<int64_t>(G, 1), true));
+    return kDataOff + skinny_data_bytes_upto(std::max<int64_t>(batch, 1), std::max<int64_t>(G, 1),
+                                             std::max<int64_t>(G, 1), true);
 }
 
 int dels_gru_step(const void* gi_table, int64_t ld_gi, int64_t table_rows, const int64_t* tokens,
@@ -1118,10 +1122,12 @@ int dels_gru_step(const void* gi_table, int64_t ld_gi, int64_t table_rows, const
 
 size_t dels_rollout_ws_bytes(int64_t batch, int64_t G, int64_t r, int64_t V) {
     if (!rows_ok(batch) || !rows_ok(G) || !rows_ok(r) || !vocab_ok(V)) return 0;
-    const size_t total = rollout_layout(std::max<int64_t>(batch, 1), std::max<int64_t>(G, 1), std::max<int64_t>(r, 1),
-                                        std::max<int64_t>(V, 1)).total;
-    // room for the one-launch rollout of two row groups where the batch may take it
-    return batch > 16 && batch <= 32 && r == kResidentRank ? std::max(total, kDataOff + kResident2Bytes) : total;
+    batch = std::max<int64_t>(batch, 1), G = std::max<int64_t>(G, 1), r = std::max<int64_t>(r, 1);
+    const size_t total = kDataOff + std::max(skinny_data_bytes_upto(batch, G, r, false),
+                                             skinny_data_bytes_upto(batch, G, G, true)) +
+                         align256(argmax_data_bytes(batch, r, std::max<int64_t>(V, 1)));
+    // room for the one-launch rollout of two row groups (17 to 32 rows)
+    return batch > 16 && r == kResidentRank ? std::max(total, kDataOff + kResident2Bytes) : total;
 }
 
 int dels_rollout_enqueue(const dels_rollout* p, void* stream) {
@@ -1253,8 +1259,11 @@ size_t dels_domino_rollout_ws_bytes(int64_t batch, int64_t steps, int64_t D, int
     if (!rows_ok(batch) || !rows_ok(steps) || !rows_ok(batch * steps) || !inner_ok(D) || !rows_ok(G) ||
         !rows_ok(E) || !vocab_ok(V))
         return 0;
-    return domino_layout(std::max<int64_t>(batch, 1), std::max<int64_t>(steps, 1), std::max<int64_t>(D, 1),
-                         std::max<int64_t>(G, 1), std::max<int64_t>(E, 1)).total;
+    batch = std::max<int64_t>(batch, 1), steps = std::max<int64_t>(steps, 1), D = std::max<int64_t>(D, 1);
+    G = std::max<int64_t>(G, 1), E = std::max<int64_t>(E, 1);
+    return kDataOff + std::max(skinny_data_bytes_upto(batch * steps, D, E, false),
+                               std::max(skinny_data_bytes_upto(batch, G, E, false),
+                                        skinny_data_bytes_upto(batch, G, G, true)));
 }
 
 int dels_domino_rollout_enqueue(const dels_domino_rollout* p, void* stream) {

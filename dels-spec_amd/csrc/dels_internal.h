@@ -81,6 +81,9 @@ struct SkinnyPlan {
 SkinnyPlan plan_skinny(int64_t rows, int64_t K, int64_t cols, bool gru);
 // Bytes of the data region the plan needs (its counters live in the control area).
 size_t skinny_data_bytes(const SkinnyPlan& p);
+// The most of it that any number of rows up to `rows` takes: what the size
+// queries answer, so that a workspace made for some rows serves fewer.
+size_t skinny_data_bytes_upto(int64_t rows, int64_t K, int64_t cols, bool gru);
 bool skinny_supported(const SkinnyPlan& p);
 
 struct RankArgs {

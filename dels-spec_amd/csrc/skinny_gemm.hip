@@ -649,7 +649,7 @@ SkinnyPlan plan_skinny(int64_t rows, int64_t K, int64_t cols, bool gru) {
         int ks = tiles >= 256 ? 1 : rows <= 32 ? 16 : 8;
         ks = std::min(ks, std::max(1, nchunks / 2));
         p.ksplit = std::min(ks, kMaxKSplit);
-        // (never less than 64 rows' 8 splits: a workspace made for more rows serves fewer)
+        // (never less than 64 rows' 8 splits, so that up to 64 rows more rows need no less)
         const int64_t prows = std::max<int64_t>(p.ksplit * rows, rows < kRankTiledMinRowsShortK ? 512 : 0);
         p.partial_bytes = p.ksplit > 1 ? (size_t)prows * cols * sizeof(float) : 0;
         return p;
@@ -681,6 +681,32 @@ SkinnyPlan plan_skinny(int64_t rows, int64_t K, int64_t cols, bool gru) {
 }
 
 size_t skinny_data_bytes(const SkinnyPlan& p) { return align256(p.partial_bytes); }
+
+// The partials fall where a plan ends splitting K (the tiles alone fill the
+// device), so the row counts tried are the ends of the ranges in which they grow.
+size_t skinny_data_bytes_upto(int64_t rows, int64_t K, int64_t cols, bool gru) {
+    size_t most = 0;
+    auto at = [&](int64_t r) {
+        if (r >= 1) most = std::max(most, skinny_data_bytes(plan_skinny(std::min(rows, r), K, cols, gru)));
+    };
+    at(rows);
+    at(16);
+    if (gru) {   // 16, 32 or 64 rows per tile
+        at(32);
+        at(64);
+        return most;
+    }
+    if (K <= kRankWholeK && rows < kRankTiledMinRowsShortK) return most;   // K whole
+    if (K % kRgChunk == 0 && cols % 8 == 0) {
+        const int64_t fit = 255 / cdiv(cols, 64);   // row tiles that leave K split
+        at(kRankTiledMinRowsShortK - 1);
+        at(std::min<int64_t>(255, 64 * fit));
+        at(128 * fit);
+    } else {
+        for (int64_t m = 1; 32 * (m - 1) < rows && m * cdiv(cols, 32) <= 128; ++m) at(32 * m);
+    }
+    return most;
+}
 
 bool skinny_supported(const SkinnyPlan& p) { return (int64_t)p.m_wg * p.n_wg <= kMaxCounters; }
 

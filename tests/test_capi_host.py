@@ -272,3 +272,25 @@ def test_golden_fixtures_reproduce_from_oracle():
         assert set(want.files) == set(got), name
         for k in want.files:
             np.testing.assert_array_equal(want[k], got[k], err_msg=f"{name}:{k}")
+
+
+def test_workspace_sizes_never_shrink_with_more_rows(pkg):
+    """A workspace made for some number of rows serves every smaller one: the size queries do not fall
+    where a kernel of more rows needs less (its tiles alone fill the device, K is not split)."""
+    lib = pkg._lib.load()
+    rows = list(range(1, 600)) + list(range(600, 4200, 37)) + [3968, 3969, 4096, 8192, 20000]
+    rows.sort()
+    for d, r in ((4096, 512), (4096, 8192), (4096, 4096), (2560, 256), (2048, 8192), (1024, 512), (4104, 512),
+                 (4096, 520), (4100 * 8, 24), (2112, 1 << 14)):
+        for size in (lambda m: lib.dels_rank_proj_ws_bytes(m, d, r),
+                     lambda m: lib.dels_lowrank_argmax_ws_bytes(m, d, r, 151936),
+                     lambda m: lib.dels_lowrank_argmax_fp8_ws_bytes(m, d, r, 151936),
+                     lambda m: lib.dels_domino_rollout_ws_bytes(1, m, d, 1024, r, 151936)):
+            got = [size(m) for m in rows]
+            assert all(a <= b for a, b in zip(got, got[1:])), (d, r)
+    for G in (64, 512, 1024, 2048, 4096, 2056):
+        for r in (128, 256, 512):
+            got = [lib.dels_rollout_ws_bytes(b, G, r, 151936) for b in range(1, 65)]
+            assert got == sorted(got), (G, r)
+        got = [lib.dels_gru_step_ws_bytes(b, G) for b in range(1, 65)]
+        assert got == sorted(got), G
