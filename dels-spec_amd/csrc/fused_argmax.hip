@@ -47,8 +47,12 @@ bool tiled_eligible(const ArgmaxArgs& a) {
 // V = 151936, per step of a rollout: 43.9 us, 38.0 us here).
 constexpr int kRowsMinRows = 17;
 
+// (V >= 4: the kernels' loads are of whole quads of columns)
 bool rows_eligible(const ArgmaxArgs& a, int prior_kind) {
-    return a.M >= kRowsMinRows && rows_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+    return a.M >= kRowsMinRows && a.V >= 4 && rows_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+}
+bool rows8_eligible(const ArgmaxArgs& a, int prior_kind) {
+    return a.M >= kRowsMinRows && a.V >= 4 && rows8_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
 }
 
 // Four-element loads of base and prior: aligned rows of whole quads, and byte
@@ -388,7 +392,7 @@ hipError_t launch_fused_argmax_fp8(const ArgmaxArgs& a, void* ws, size_t data_of
     ka.counter = reinterpret_cast<unsigned int*>(w + kCountersOff);
     ka.keys = reinterpret_cast<unsigned long long*>(w + kKeysOff);
     ka.key_stride = (int64_t)a.M * 128 <= (int64_t)(kCtrlBytes - kKeysOff) ? 16 : 1;
-    if (a.M >= kRowsMinRows && rows8_rank_ok(a.r) && rows_prior_ok(a.base_dtype, pk)) {
+    if (rows8_eligible(a, pk)) {
         const bool vec = rows8_vec(a);
         if (a.base_dtype == 1) return launch_rows8_bf16(ka, pk, vec, s);
         if (a.base_dtype == 2) return launch_rows8_f16(ka, pk, vec, s);

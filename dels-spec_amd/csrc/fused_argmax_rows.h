@@ -17,13 +17,16 @@
 // matrix cores are each busy for 8 of the ~27 us the stream takes), which leaves
 // the registers to the stream: two waves per SIMD with two tiles each in flight.
 // (With the operands in registers, one wave per SIMD: 40 / 48 rows 38.5 / 39.7
-// us a launch, 33.9 / 34.7 here at r = 512, V = 151936; 64 rows of an unaligned
-// vocabulary of 50257, 37.5 and 27.1; 40 rows in the GEMV kernel, 104.)  The
+// us a launch, 33.9 / 34.7 here at r = 512, V = 151936; 40 rows in the GEMV
+// kernel, 104.)  The
 // tile is the MFMA's A operand and the rank its B operand: lane l ends with row
 // l % 16 of each group and the four consecutive columns 4 (l / 16) .. + 3, so
 // that a lane's base logits are one 8- or 16-byte load per group, its prior
 // values one load for all groups, and the running argmax takes one (score,
-// index) pair per group.  Tiles are walked wave-strided through two register
+// index) pair per group.  Unaligned rows and vocabularies take the same loads
+// at element alignment (load_quad_any: with four element loads instead, 63 rows
+// at V = 50257 took 18.5 / 21.2 / 26.8 us at r = 128 / 256 / 512, more than the
+// GEMV kernel's 13.8 / 17.4 / 24.8; as quads 11.7 / 14.2 / 18.3).  Tiles are walked wave-strided through two register
 // sets, refills unconditional, as in the GEMV kernel.
 #pragma once
 
@@ -39,18 +42,55 @@ namespace rows {
 constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 
-// Values a lane takes from a row per tile: four consecutive ones.  VEC: as one
-// load (two words of 16-bit values, four of fp32), else four element loads.
-template <typename T, bool VEC>
-constexpr int quad_words() { return VEC && sizeof(T) == 2 ? 2 : 4; }
+// The four consecutive values a lane takes from a row per tile, as loaded: two
+// words of 16-bit values, four of fp32.
+template <typename T>
+constexpr int quad_words() { return sizeof(T) == 2 ? 2 : 4; }
+template <typename T>
+using Quad = uint32_t[quad_words<T>()];
 
 // Row offsets (bytes) fit 32 bits with VEC, so that a row costs one register.
 template <bool VEC>
 using RowOff = typename std::conditional<VEC, uint32_t, int64_t>::type;
 
+// Columns v .. v + 3 of a row of four or more, at any alignment: one load at
+// element alignment, taken back into the row at its end (shift_quad puts its
+// elements in place when it is used).  Four element loads instead touch each of
+// a wave's 16 rows four times.
+template <typename T>
+__device__ __forceinline__ void load_quad_any(const T* row, int v, int V, Quad<T>& w) {
+    const T* p = row + min(v, V - 4);
+    if constexpr (sizeof(T) == 2) {
+        typedef uint64_t __attribute__((aligned(2))) u64_a2;
+        const uint64_t x = *reinterpret_cast<const u64_a2*>(p);
+        w[0] = (uint32_t)x; w[1] = (uint32_t)(x >> 32);
+    } else {
+        typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
+        const u32x4 x = *reinterpret_cast<const u32x4_a4*>(p);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) w[q] = x[q];
+    }
+}
+
+// The quad of columns v .. v + 3 from one that was taken back to V - 4 (columns
+// past V are not used).
+template <typename T>
+__device__ __forceinline__ void shift_quad(Quad<T>& w, int v, int V) {
+    const int d = V >= 4 ? min(max(v - (V - 4), 0), 3) : 0;
+    if constexpr (sizeof(T) == 2) {
+        const uint64_t x = (((uint64_t)w[1] << 32) | w[0]) >> (16 * d);
+        w[0] = (uint32_t)x; w[1] = (uint32_t)(x >> 32);
+    } else {
+#pragma unroll
+        for (int q = 0; q < 3; ++q)
+#pragma unroll
+            for (int o = 1; q + o < 4; ++o) w[q] = d == o ? w[q + o] : w[q];
+    }
+}
+
+// VEC: aligned quads, V a multiple of 4.
 template <typename T, bool VEC>
-__device__ __forceinline__ void load_quad(const void* base, RowOff<VEC> row, int v, int V,
-                                          uint32_t (&w)[quad_words<T, VEC>()]) {
+__device__ __forceinline__ void load_quad(const void* base, RowOff<VEC> row, int v, int V, Quad<T>& w) {
     const char* p = static_cast<const char*>(base);
     if constexpr (VEC) {
         const uint32_t o = row + (uint32_t)min(v, V - 4) * (uint32_t)sizeof(T);   // V a multiple of 4: whole quads
@@ -63,16 +103,14 @@ __device__ __forceinline__ void load_quad(const void* base, RowOff<VEC> row, int
             for (int q = 0; q < 4; ++q) w[q] = x[q];
         }
     } else {
-        const T* r = reinterpret_cast<const T*>(p + row);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] = load_raw(r + min(v + q, V - 1));
+        load_quad_any<T>(reinterpret_cast<const T*>(p + row), v, V, w);
     }
 }
 
 // Value q of a quad, widened.
-template <typename T, bool VEC>
-__device__ __forceinline__ float quad_at(const uint32_t (&w)[quad_words<T, VEC>()], int q) {
-    if constexpr (VEC && sizeof(T) == 2) return tiled::half_at<T>(w[q >> 1], q & 1);
+template <typename T>
+__device__ __forceinline__ float quad_at(const Quad<T>& w, int q) {
+    if constexpr (sizeof(T) == 2) return tiled::half_at<T>(w[q >> 1], q & 1);
     else return widen_raw<T>(w[q]);
 }
 
@@ -81,11 +119,11 @@ __device__ __forceinline__ float quad_at(const uint32_t (&w)[quad_words<T, VEC>(
 // Ranks the kernel takes: whole MFMA K steps, no masked operands.
 inline bool rows_rank_ok(int r) { return r == 128 || r == 256 || r == 512; }
 
-template <int RG, int KSTEPS, typename BaseT, typename PriorT, bool VEC>
+template <int RG, int KSTEPS, typename BaseT, typename PriorT>
 struct RowsTile {
     bf16x8 b[KSTEPS];
-    uint32_t base[RG][rows::quad_words<BaseT, VEC>()];
-    uint32_t prior[rows::quad_words<PriorT, VEC>()];
+    rows::Quad<BaseT> base[RG];
+    rows::Quad<PriorT> prior;
 };
 
 // End of a workgroup's share of the argmax over the rows m0 .. m0 + 16 RG - 1:
@@ -182,7 +220,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(Argma
         bidx[g] = INT_MAX;
     }
 
-    using Tile = RowsTile<RG, KSTEPS, BaseT, PriorT, VEC>;
+    using Tile = RowsTile<RG, KSTEPS, BaseT, PriorT>;
     // live (uniform) false: not one of the wave's tiles -- the same loads, of one line each
     auto load = [&](int t, bool live, Tile& tr) {
         // ROWMAJOR: the lane's K octets of vocabulary row t * 16 + col; else MFMA-16 blocks
@@ -195,7 +233,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(Argma
         for (int g = 0; g < RG; ++g) load_quad<BaseT, VEC>(a.base, live ? brow[g] : 0, v, a.V, tr.base[g]);
         if constexpr (HAS_PRIOR) load_quad<PriorT, VEC>(a.prior, 0, v, a.V, tr.prior);
     };
-    auto consume = [&](const Tile& tr, int t) {
+    auto consume = [&](Tile& tr, int t) {
         // the operands are read from LDS tile by tile: through the empty asm statement the
         // compiler cannot take them for loop invariants and hold them in registers
         int lo = lane * 16;
@@ -210,14 +248,21 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows_kernel(Argma
                 acc[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
                     tr.b[s], *reinterpret_cast<const bf16x8*>(s_rank + (s * RG + g) * 1024 + lo), acc[g], 0, 0, 0);
         const int v = t * 16 + 4 * kg;
+        if constexpr (!VEC) {
+            if (t * 16 + 16 > a.V) {   // wave-uniform
+#pragma unroll
+                for (int g = 0; g < RG; ++g) shift_quad<BaseT>(tr.base[g], v, a.V);
+                if constexpr (HAS_PRIOR) shift_quad<PriorT>(tr.prior, v, a.V);
+            }
+        }
 #pragma unroll
         for (int q = 3; q >= 0; --q) {
             const bool in = v + q < a.V;
             float pv = 0.f;
-            if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
+            if constexpr (HAS_PRIOR) pv = quad_at<PriorT>(tr.prior, q);
 #pragma unroll
             for (int g = 0; g < RG; ++g) {
-                float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT, VEC>(tr.base[g], q));
+                float sc = __builtin_fmaf(acc[g][q], al[g], quad_at<BaseT>(tr.base[g], q));
                 if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
                 // a lane's candidates arrive in decreasing column order: ">=" ends at the lowest index,
                 // that of a first score of -inf among them

@@ -26,12 +26,12 @@
 
 namespace dels {
 
-template <int RG, int KS8, typename BaseT, typename PriorT, bool VEC>
+template <int RG, int KS8, typename BaseT, typename PriorT>
 struct Rows8Tile {
     i32x8 b[KS8];
-    uint32_t base[RG][rows::quad_words<BaseT, VEC>()];
-    uint32_t prior[rows::quad_words<PriorT, VEC>()];
-    uint32_t bscale[4];
+    rows::Quad<BaseT> base[RG];
+    rows::Quad<PriorT> prior;
+    rows::Quad<float> bscale;
 };
 
 // HAS_PRIOR false: the prior term is absent (PriorT is then BaseT and unused).
@@ -40,7 +40,8 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
 #pragma clang fp contract(off)
     using namespace rows;
     constexpr int kRows = 16 * RG;
-    constexpr int kND = 3;                                    // tiles in flight per wave
+    // tiles in flight per wave: three where they fit the registers
+    constexpr int kND = !VEC && RG == 4 && sizeof(BaseT) == 4 ? 2 : 3;
     extern __shared__ __attribute__((aligned(16))) char s_rank[];   // [KS8][RG][2][64 lanes][16 bytes]
     __shared__ float s_rsc[kRows];
     __shared__ float s_val[kWaves][kRows];
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
     }
     asm volatile("" ::: "memory");   // these loads stay ahead of the stream's
 
-    using Tile = Rows8Tile<RG, KS8, BaseT, PriorT, VEC>;
+    using Tile = Rows8Tile<RG, KS8, BaseT, PriorT>;
     // live (uniform) false: not one of the wave's tiles -- the same loads, of one line each
     auto load = [&](int t, bool live, Tile& tr) {
         const uint8_t* bp = reinterpret_cast<const uint8_t*>(a.B) + (int64_t)t * KS8 * kFp8K128Block + (live ? lane * 16 : 0);
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
         load_quad<float, VEC>(a.b_scale, 0, v, a.V, tr.bscale);
     };
     float rsc[RG];
-    auto consume = [&](const Tile& tr, int t) {
+    auto consume = [&](Tile& tr, int t) {
         // operands tile by tile from LDS (see the bf16 kernel)
         int lo = lane * 16;
         asm volatile("" : "+v"(lo));
@@ -118,17 +119,23 @@ __global__ __launch_bounds__(rows::kThreads) void fused_argmax_rows8_kernel(Argm
                                                             (int)y[1], (int)y[2], (int)y[3]}, acc[g]);
             }
         const int v = t * 16 + 4 * kg;
+        if constexpr (!VEC) {
+#pragma unroll
+            for (int g = 0; g < RG; ++g) shift_quad<BaseT>(tr.base[g], v, a.V);
+            if constexpr (HAS_PRIOR) shift_quad<PriorT>(tr.prior, v, a.V);
+            shift_quad<float>(tr.bscale, v, a.V);
+        }
 #pragma unroll
         for (int q = 3; q >= 0; --q) {
             const bool in = v + q < a.V;
             const float bs = __uint_as_float(tr.bscale[q]);
             float pv = 0.f;
-            if constexpr (HAS_PRIOR) pv = quad_at<PriorT, VEC>(tr.prior, q);
+            if constexpr (HAS_PRIOR) pv = quad_at<PriorT>(tr.prior, q);
 #pragma unroll
             for (int g = 0; g < RG; ++g) {
                 float dot = acc[g][q] * rsc[g];
                 dot = dot * bs;
-                float sc = __builtin_fmaf(dot, al[g], quad_at<BaseT, VEC>(tr.base[g], q));
+                float sc = __builtin_fmaf(dot, al[g], quad_at<BaseT>(tr.base[g], q));
                 if constexpr (HAS_PRIOR) sc = use_prior[g] ? __builtin_fmaf(nbe[g], pv, sc) : sc;
                 // a lane's candidates arrive in decreasing column order: ">=" ends at the lowest index,
                 // that of a first score of -inf among them

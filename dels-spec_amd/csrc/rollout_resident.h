@@ -185,9 +185,7 @@ constexpr int kRrPriorWords = kRrPriorZeros + 16;
 // aligned to four elements.  (Element loads take a line per row each: twenty of
 // them per lane and group made a vocabulary of 50257 slower than one of 151936.)
 template <typename BaseT>
-using RrQuad = uint32_t[rows::quad_words<BaseT, true>()];
-template <typename BaseT>
-using RrBase = RrQuad<BaseT>[kRrRegTiles + 1];
+using RrBase = rows::Quad<BaseT>[kRrRegTiles + 1];
 
 // `row`: the lane's row of the step.  Tiles past the workgroup's repeat its last one.
 template <typename BaseT, bool VEC>
@@ -208,19 +206,7 @@ __device__ __forceinline__ void rr_load_base(const BaseT* row, int T0, int ntl, 
                 for (int q = 0; q < 4; ++q) w[j][q] = x[q];
             }
         } else if (V >= 4) {
-            // elsewhere a quad is one load at element alignment, taken back into the
-            // row at its end (rr_shift_quad puts its elements in place when it is used)
-            const BaseT* p = row + min(v, V - 4);
-            if constexpr (sizeof(BaseT) == 2) {
-                typedef uint64_t __attribute__((aligned(2))) u64_a2;
-                const uint64_t x = *reinterpret_cast<const u64_a2*>(p);
-                w[j][0] = (uint32_t)x; w[j][1] = (uint32_t)(x >> 32);
-            } else {
-                typedef u32x4 __attribute__((aligned(4))) u32x4_a4;
-                const u32x4 x = *reinterpret_cast<const u32x4_a4*>(p);
-#pragma unroll
-                for (int q = 0; q < 4; ++q) w[j][q] = x[q];
-            }
+            rows::load_quad_any<BaseT>(row, v, V, w[j]);
         } else {
             uint32_t e[4];
 #pragma unroll
@@ -233,22 +219,6 @@ __device__ __forceinline__ void rr_load_base(const BaseT* row, int T0, int ntl, 
                 for (int q = 0; q < 4; ++q) w[j][q] = e[q];
             }
         }
-    }
-}
-
-// The quad of columns v .. v + 3 from one that was taken back to V - 4 (columns
-// past V are not used).
-template <typename BaseT>
-__device__ __forceinline__ void rr_shift_quad(RrQuad<BaseT>& w, int v, int V) {
-    const int d = V >= 4 ? min(max(v - (V - 4), 0), 3) : 0;
-    if constexpr (sizeof(BaseT) == 2) {
-        const uint64_t x = (((uint64_t)w[1] << 32) | w[0]) >> (16 * d);
-        w[0] = (uint32_t)x; w[1] = (uint32_t)(x >> 32);
-    } else {
-#pragma unroll
-        for (int q = 0; q < 3; ++q)
-#pragma unroll
-            for (int o = 1; q + o < 4; ++o) w[q] = d == o ? w[q + o] : w[q];
     }
 }
 
@@ -297,14 +267,14 @@ __device__ __forceinline__ unsigned long long rr_tiles_best(const bf16x8 (&bt)[k
         const int tc = min(ti, max(ntl - 1, 0));
         const int left = live ? V - (T0 + tc) * 16 - 4 * kg : 0;   // columns from the lane's first one on
         if constexpr (!VEC)
-            if ((T0 + tc) * 16 + 16 > V) rr_shift_quad<BaseT>(braw[j], (T0 + tc) * 16 + 4 * kg, V);   // wave-uniform
+            if ((T0 + tc) * 16 + 16 > V) rows::shift_quad<BaseT>(braw[j], (T0 + tc) * 16 + 4 * kg, V);   // wave-uniform
         f32x4 pv = {0.f, 0.f, 0.f, 0.f};
         if constexpr (!is_no_prior<PriorT>::value)
             pv = *reinterpret_cast<const f32x4*>(s_prior + (be != 0.f ? tc * 16 : kRrPriorZeros) + 4 * kg);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const float al_q = (VEC ? 0 : q) < left ? al : nan;
-            float sc = __builtin_fmaf(acc[j][q], al_q, rows::quad_at<BaseT, true>(braw[j], q));
+            float sc = __builtin_fmaf(acc[j][q], al_q, rows::quad_at<BaseT>(braw[j], q));
             if constexpr (!is_no_prior<PriorT>::value) sc = __builtin_fmaf(-be, pv[q], sc);
             acc[j][q] = sc;
             best = __builtin_fmaxf(best, sc);

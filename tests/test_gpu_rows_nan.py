@@ -18,6 +18,7 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
     (33, 20011, F32, None),           # element loads
     (40, 16, BF16, None),             # one tile for the whole grid
     (20, 5, F16, F32),                # less than a tile
+    (18, 3, BF16, None),              # less than a quad
     (63, 70000, F16, F16),            # several tiles per wave
     (70, 9003, BF16, BF16),           # past 64 rows where the tiled kernel does not apply
 ])
