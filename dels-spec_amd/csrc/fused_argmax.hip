@@ -47,12 +47,39 @@ bool tiled_eligible(const ArgmaxArgs& a) {
 // V = 151936, per step of a rollout: 43.9 us, 38.0 us here).
 constexpr int kRowsMinRows = 17;
 
-// (V >= 4: the kernels' loads are of whole quads of columns)
-bool rows_eligible(const ArgmaxArgs& a, int prior_kind) {
-    return a.M >= kRowsMinRows && a.V >= 4 && rows_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+// Vocabulary from which it pays.  A short B lies in the caches, where a second
+// pass costs little, while the sharing kernel fills its LDS with the rank
+// operands first (16 to 64 KiB per workgroup) and has a workgroup per 128
+// columns.  GEMV / sharing kernel, bf16: V = 2000, r = 512, 24 rows 7.7 / 8.6 us,
+// 63 rows 8.7 / 11.8, r = 256, 63 rows 7.6 / 8.9; V = 4000, r = 512, 40 rows 9.4
+// / 10.2; V = 8192, r = 512, 24 rows 10.1 / 8.9, 63 rows 11.0 / 12.2; V = 12000,
+// 63 rows 12.8 / 12.6; V = 8192, r = 256, 40 rows 9.1 / 8.8.  Past 64 rows, where
+// the GEMV kernel's passes are five and more, it pays sooner (row-major, fp32 base,
+// r = 512, V = 4000, 200 rows 25.7 / 14.7).  (The sharing kernels load whole quads
+// of columns: never below 4.)
+bool rows_vocab_pays(const ArgmaxArgs& a) {
+    return a.V >= std::max(3072, (a.M <= 48 ? 16 : a.M <= 64 ? 20 : 6) * a.r);
 }
+
+bool rows_eligible(const ArgmaxArgs& a, int prior_kind) {
+    return a.M >= kRowsMinRows && rows_vocab_pays(a) && rows_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+}
+
+// The e4m3 form: B is half as long and, with three tiles in flight per wave, a
+// vocabulary below about 36000 leaves its waves a tile or less, so that up to
+// there it pays only where the GEMV kernel's passes are two (V = 8192, r = 256,
+// 24 rows 9.8 / 7.8 us), more than four or, at r = 512, three (V = 16384, 40 rows
+// 15.3 / 12.3): r = 256, V = 32000, 40 rows 12.1 / 12.8; r = 512, 63 rows, V =
+// 16384 12.1 / 12.4, V = 40000 16.1 / 14.9.  Of two passes it is no better from
+// about 28000 on, where every wave has one tile and none a second to overlap
+// (V = 32001, 24 rows 10.8 / 11.6 at r = 256).
+constexpr int kRows8AnyVocab = 36864;
+constexpr int kRows8TwoPassVocab = 28672;
 bool rows8_eligible(const ArgmaxArgs& a, int prior_kind) {
-    return a.M >= kRowsMinRows && a.V >= 4 && rows8_rank_ok(a.r) && rows_prior_ok(a.base_dtype, prior_kind);
+    if (a.M < kRowsMinRows || !rows8_rank_ok(a.r) || !rows_prior_ok(a.base_dtype, prior_kind)) return false;
+    if (!rows_vocab_pays(a)) return false;
+    if (a.V >= kRows8AnyVocab || a.M > 64) return true;
+    return a.M <= 32 ? a.V < kRows8TwoPassVocab : a.M <= 48 && a.r == 512;
 }
 
 // Four-element loads of base and prior: aligned rows of whole quads, and byte

@@ -26,8 +26,9 @@
 // index) pair per group.  Unaligned rows and vocabularies take the same loads
 // at element alignment (load_quad_any: with four element loads instead, 63 rows
 // at V = 50257 took 18.5 / 21.2 / 26.8 us at r = 128 / 256 / 512, more than the
-// GEMV kernel's 13.8 / 17.4 / 24.8; as quads 11.7 / 14.2 / 18.3).  Tiles are walked wave-strided through two register
-// sets, refills unconditional, as in the GEMV kernel.
+// GEMV kernel's 13.8 / 17.4 / 24.8; as quads 11.7 / 14.2 / 18.3).  Tiles are
+// walked wave-strided through two register sets, refills unconditional, as in the
+// GEMV kernel.
 #pragma once
 
 #include <mutex>
@@ -347,13 +348,16 @@ hipError_t launch_rows_for_base(const ArgmaxKArgs& ka, bool packed, int prior_ki
             constexpr bool RM = decltype(rm_tag)::value;
             if (ka.M <= 32) return launch_rows_inst<2, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
             // three groups where their operands split evenly over the threads; eight, past
-            // 64 rows, where their base logits fit the registers (200 rows, row-major:
-            // 141 us with four, 114 with eight)
+            // 64 rows, where their base logits fit the registers and B is long (200 rows,
+            // row-major, r = 512, V = 151936: 141 us with four, 114 with eight; on a short
+            // one the longer fill of the LDS is not made up: 80 rows, V = 24000, r = 256, 13 %
+            // more with eight; V = 65536, 3 % less, at r = 128 13 % more; V = 128000 10 % less)
             if constexpr (VEC) {
                 if constexpr (KS >= 8)
                     if (ka.M <= 48) return launch_rows_inst<3, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
                 if constexpr (sizeof(BaseT) == 2)
-                    if (ka.M > 64) return launch_rows_inst<8, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
+                    if (ka.M > 64 && ka.V >= (KS >= 8 ? 49152 : 114688))
+                        return launch_rows_inst<8, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
             }
             return launch_rows_inst<4, KS, RM, BaseT, PriorT, VEC, HP>(ka, s);
         };

@@ -15,12 +15,13 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 @pytest.mark.parametrize("fmt", ["packed", "rowmajor", "e4m3"])
 @pytest.mark.parametrize("M,V,bdt,pdt", [
     (17, 4112, BF16, BF16),
-    (33, 20011, F32, None),           # element loads
-    (40, 16, BF16, None),             # one tile for the whole grid
-    (20, 5, F16, F32),                # less than a tile
+    (33, 40011, F32, None),           # unaligned rows
+    (32, 4097, F16, F32),             # one column in the last tile
+    (49, 36867, BF16, BF16),          # less than a quad of columns in the last tile
     (18, 3, BF16, None),              # less than a quad
     (63, 70000, F16, F16),            # several tiles per wave
     (70, 9003, BF16, BF16),           # past 64 rows where the tiled kernel does not apply
+    (131, 65540, BF16, F32),          # ... eight groups a pass
 ])
 def test_rows_of_nan_and_inf(pkg, dev, fmt, M, V, bdt, pdt):
     print(f"case rows nan M={M} V={V} base={bdt} prior={pdt} {fmt}", flush=True)
