@@ -262,7 +262,8 @@ static int enqueue_rollout(const dels_rollout* p, hipStream_t s) {
     uint16_t* h_next = static_cast<uint16_t*>(p->h_b);
     const size_t esz = dtype_size(p->base_dtype);
     const bool packed = p->weights_layout == DELS_LAYOUT_MFMA16;
-    if (rollout_resident_enabled() && rollout_resident_eligible(B, G, r, V, p->steps, packed, p->ws_bytes)) {
+    if (rollout_resident_enabled() && rollout_resident_eligible(B, G, r, V, p->steps, packed, p->ws_bytes) &&
+        (rollout_resident_forced() || rollout_resident_pays(B, V, p->steps))) {
         // every step in one launch with B held on chip (rollout_resident.hip)
         ResidentRolloutArgs ra{};
         ra.w_hh = g.w_hh; ra.b_hh = g.b_hh;
@@ -445,7 +446,8 @@ static int enqueue_markov(const dels_markov_rollout* p, hipStream_t s) {
     const int64_t ldbase = p->ld_base ? p->ld_base : p->steps * p->V;
     const bool packed = p->lm_layout == DELS_LAYOUT_MFMA16;
     if (rollout_resident_enabled() &&
-        markov_resident_eligible(p->batch, p->r, p->V, p->steps, packed, p->ws_bytes)) {
+        markov_resident_eligible(p->batch, p->r, p->V, p->steps, packed, p->ws_bytes) &&
+        (rollout_resident_forced() || markov_resident_pays(p->batch, p->V, p->steps))) {
         // every step in one launch with B held on chip (markov_resident.hip)
         MarkovRolloutArgs a{};
         a.embedding = static_cast<const uint16_t*>(p->embedding);

@@ -221,8 +221,10 @@ hipError_t launch_rollout_ordered(const ResidentRolloutArgs& a, void* ws, hipStr
 int resident_spin_limit();
 int set_resident_spin_limit(int limit);   // returns the previous limit
 void set_ordered_wait_limit(int limit);   // < 0: the default
-int set_rollout_resident(int enable);   // returns the previous setting (1 = used where eligible)
+int set_rollout_resident(int enable);   // returns the previous setting (1 = used where eligible and it pays)
 bool rollout_resident_enabled();
+bool rollout_resident_forced();          // used wherever eligible
+bool rollout_resident_pays(int64_t batch, int64_t V, int64_t steps);
 // The Markov rollout with B resident on chip (markov_resident.hip: r = 128 or
 // 256, batch <= 32), followed on the stream by the ordered rollout, which does
 // the work when the resident launch could not get every CU and returns at once
@@ -248,6 +250,7 @@ struct MarkovRolloutArgs {
 // rollout keeps its state words.
 constexpr size_t kMarkovSlotBytes = align256((size_t)4 * 16 * kResidentMaxWGs * 8);
 bool markov_resident_eligible(int64_t batch, int64_t r, int64_t V, int64_t steps, bool packed, size_t ws_bytes);
+bool markov_resident_pays(int64_t batch, int64_t V, int64_t steps);
 hipError_t launch_markov_resident(MarkovRolloutArgs a, void* ws, hipStream_t s);
 hipError_t launch_markov_ordered(const MarkovRolloutArgs& a, hipStream_t s);
 // The fp8 decode step (A e4m3 K32, B e4m3 K128): as above with r in {128, 256, 512}.

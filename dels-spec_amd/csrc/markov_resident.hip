@@ -270,6 +270,18 @@ bool markov_resident_eligible(int64_t batch, int64_t r, int64_t V, int64_t steps
     return (ntiles + nwg - 1) / nwg <= kRrWaves * kRrRegTiles + kResidentLdsTiles;
 }
 
+// One launch takes 13 to 21 us before its first step (B on chip, everyone's
+// arrival, the stand-in behind it) and about 5 a step (two groups of rows 8), the
+// per-step launches 6 and as much a step as the vocabulary asks: at V = 2000 /
+// 8192 / 16384 / 32000 / 65536 / 151936, r = 256, 16 rows 6.4 / 7.7 / 10.2 / 10.6
+// / 13.1 / 18.5, 32 rows 7.0 / 7.3 / 8.5 / 10.8 / 13.6 / 18.5.  The steps from
+// which one launch is ahead (r = 128 differs little); below the last line it never
+// was in 24 steps of two groups.
+bool markov_resident_pays(int64_t batch, int64_t V, int64_t steps) {
+    if (batch <= 16) return steps >= (V >= 65536 ? 2 : V >= 32768 ? 3 : V >= 16384 ? 4 : V >= 8192 ? 8 : 16);
+    return V >= 30720 && steps >= (V >= 98304 ? 3 : V >= 65536 ? 4 : 8);
+}
+
 hipError_t launch_markov_resident(MarkovRolloutArgs a, void* ws, hipStream_t s) {
     char* w = static_cast<char*>(ws);
     a.ntiles = (a.V + 15) / 16;

@@ -577,12 +577,22 @@ int set_resident_spin_limit(int limit) {
     g_resident_spin_limit = std::max(0, limit);
     return prev;
 }
-int set_rollout_resident(int enable) {
+int set_rollout_resident(int enable) {   // 0: off, 1: where it pays, 2: wherever it can run
     const int prev = g_resident_enabled;
-    g_resident_enabled = enable != 0;
+    g_resident_enabled = std::max(0, std::min(enable, 2));
     return prev;
 }
 bool rollout_resident_enabled() { return g_resident_enabled != 0; }
+bool rollout_resident_forced() { return g_resident_enabled > 1; }
+
+// Two groups of rows take about 18 to 25 us before their first step (B and the
+// other operands on chip) and 13 to 16 a step, the per-step launches 2 to 4 and 17
+// to 35: one step is always theirs (17 rows, G = 1024, V = 32000: 27 / 38 us), two
+// on a short vocabulary (V = 32000: 49 / 55; V = 65536 53 / 55; V = 151936 64 /
+// 57), three are even at the shortest (V = 2000: 63 / 64).
+bool rollout_resident_pays(int64_t batch, int64_t V, int64_t steps) {
+    return batch <= 16 || steps >= 3 || (steps == 2 && V >= 65536);
+}
 
 bool rollout_resident_eligible(int64_t batch, int64_t G, int64_t r, int64_t V, int64_t steps, bool packed,
                                size_t ws_bytes) {

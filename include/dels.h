@@ -222,9 +222,11 @@ int dels_debug_set_decode_spin_limit(int limit);
  * twice the CU count, the vocabulary's share fitting a CU), dels_rollout_enqueue
  * and dels_graph_create run every step of the rollout in one launch that keeps
  * the low-rank head resident on chip, and so do the Markov rollout's entry points
- * where theirs does; enable = 0 selects the per-step launches instead (for
- * later calls), 1 restores the default.  Returns the previous
- * setting.  Not thread-safe.
+ * where theirs does -- by default where that takes less time (not a Markov
+ * rollout of few steps or a short vocabulary, nor one or two steps of more than 16
+ * rows).  enable = 0 selects the per-step launches instead (for later calls), 2 the
+ * one launch wherever the shape allows it, 1 restores the default.  Returns the
+ * previous setting.  Not thread-safe.
  */
 int dels_debug_set_rollout_resident(int enable);
 /* Test hook: the waits of that one-launch rollout re-read each other's results
@@ -508,12 +510,14 @@ int dels_gather_argmax(const int64_t* tokens, int64_t tok_stride, const void* E,
  * (code/kernel/markov_dels.py:261-278): token_0 = prev_ids; for each step s,
  * out_ids[:, s] = dels_gather_argmax(token_s) against base[:, s, :] with
  * alpha[s]/beta[s], and token_{s+1} = out_ids[:, s].  With lm_w in the MFMA-16
- * layout, r = 128 or 256, batch <= 32 and a vocabulary share that fits a CU, one
- * launch that holds lm_w on chip does every step; it is followed by one that does
- * the rollout in its place when it could not get every CU of the GPU (other
- * streams or processes at work on it) and otherwise returns at once.  One launch
- * per step for other shapes, and with a workspace below
- * dels_markov_rollout_ws_bytes() that still holds the control area and words.
+ * layout, r = 128 or 256, batch <= 32, a vocabulary share that fits a CU and enough
+ * steps for the vocabulary (2 from 65536 entries on and 16 on the shortest; for
+ * more than 16 rows 3 from 98304 on, 8 from 30720 on and none below), one launch
+ * that holds lm_w on chip does every step; it is followed by one that does the
+ * rollout in its place when it could not get every CU of the GPU (other streams or
+ * processes at work on it) and otherwise returns at once.  One launch per step
+ * otherwise, and with a workspace below dels_markov_rollout_ws_bytes() that still
+ * holds the control area and words.
  */
 typedef struct dels_markov_rollout {
     const void* embedding;  /* [table_rows, r] bf16 row-major */

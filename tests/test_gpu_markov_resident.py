@@ -24,6 +24,15 @@ CASES = [
 ]
 
 
+@pytest.fixture(autouse=True)
+def _one_launch_wherever_it_can_run(pkg):
+    """Short vocabularies and few steps take the per-step launches by default."""
+    lib = pkg._lib.load()
+    was = lib.dels_debug_set_rollout_resident(2)
+    yield
+    lib.dels_debug_set_rollout_resident(was)
+
+
 class _Head(torch.nn.Module):
     def __init__(self, E, W):
         super().__init__()

@@ -20,6 +20,15 @@ BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 BETAS = [0.0, 0.25, 0.0, 0.5]
 
 
+@pytest.fixture(autouse=True)
+def _one_launch_wherever_it_can_run(pkg):
+    """Short vocabularies and few steps take the per-step launches by default."""
+    lib = pkg._lib.load()
+    was = lib.dels_debug_set_rollout_resident(2)
+    yield
+    lib.dels_debug_set_rollout_resident(was)
+
+
 def _inputs(nb, V, dt):
     """Rows of a [nb, 4, V] base: NaN up to and past tiles and quads, -inf elsewhere or everywhere, a finite
     or infinite value among them; prior -inf in a column (a -inf base there scores NaN where beta is not 0)."""

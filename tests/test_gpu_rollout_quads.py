@@ -15,6 +15,15 @@ pytestmark = pytest.mark.gpu
 BF16, F16, F32 = torch.bfloat16, torch.float16, torch.float32
 
 
+@pytest.fixture(autouse=True)
+def _one_launch_wherever_it_can_run(pkg):
+    """Short vocabularies and few steps take the per-step launches by default."""
+    lib = pkg._lib.load()
+    was = lib.dels_debug_set_rollout_resident(2)
+    yield
+    lib.dels_debug_set_rollout_resident(was)
+
+
 # vocabularies that leave 0 to 3 columns of a quad, parts of a tile, and less than a quad
 @pytest.mark.parametrize("V", [3, 5, 18, 4100, 4101, 4102, 4103])
 @pytest.mark.parametrize("dt", [BF16, F16, F32])

@@ -12,6 +12,15 @@ from test_gpu_rollout_resident import _Head as _DeLSHead
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def _one_launch_wherever_it_can_run(pkg):
+    """Short vocabularies and few steps take the per-step launches by default."""
+    lib = pkg._lib.load()
+    was = lib.dels_debug_set_rollout_resident(2)
+    yield
+    lib.dels_debug_set_rollout_resident(was)
+
+
 def _runner(pkg, dev, kind, nb, steps, V):
     sched = dict(batch_size=nb, steps=steps, vocab_size=V, alpha_values=[0.7] * steps, beta_values=[0.0] * steps,
                  baseline_logits=None, device=dev)

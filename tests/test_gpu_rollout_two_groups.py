@@ -21,6 +21,15 @@ CASES = [
 ]
 
 
+@pytest.fixture(autouse=True)
+def _one_launch_wherever_it_can_run(pkg):
+    """Short vocabularies and few steps take the per-step launches by default."""
+    lib = pkg._lib.load()
+    was = lib.dels_debug_set_rollout_resident(2)
+    yield
+    lib.dels_debug_set_rollout_resident(was)
+
+
 @torch.inference_mode()
 def _eager(runner, prefix, base):
     runner.static_prefix_ids.copy_(prefix)
