@@ -25,8 +25,9 @@
 // near 1, which is where winners are: a candidate that passes is almost always
 // a new maximum.  Everything that is compared or returned is the exact value.
 // 120 rows of 151936 bf16 logits, whole call: 65.3 -> 29.3 us, and with one wide
-// multiply per Philox product and one bitop3 per pair of xors 26.6 (18.2 M
-// candidates; their 36 MB take 7.3 us at the rate of a large copy).
+// multiply per Philox product and one bitop3 per pair of xors 26.6, with few
+// lanes at the LDS atomics 23 (18.2 M candidates; their 36 MB take 7.3 us at the
+// rate of a large copy).
 //
 // Reduction: one 64-bit key per candidate (order(score) << 32 | ~index, NaN
 // above +inf), a device-scope atomic max per workgroup into the row's key, and
@@ -91,6 +92,12 @@ template <typename T> constexpr float tempered_slack() { return 0x1p-20f; }
 template <> constexpr float tempered_slack<bf16_t>() { return 0x1p-7f; }
 template <> constexpr float tempered_slack<f16_t>() { return 0x1p-9f; }
 
+// The value of the lane K below in the DPP row of 16 lanes (0 where there is none).
+template <int K>
+__device__ __forceinline__ uint32_t row_shr(uint32_t x) {
+    return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x110 + K, 0xf, 0xf, true);
+}
+
 // Four logits as loaded: one 8- or 16-byte load where the rows allow it (VEC),
 // else four element loads, clamped to the row.
 template <typename T, bool VEC>
@@ -143,6 +150,10 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
     };
 
     unsigned long long best = 0ull;   // below every candidate's key
+    // One group per thread: no threshold would serve a later one, so every candidate
+    // is evaluated (V = 1000, one row: 6.9 us when they took bounds and a threshold
+    // too, 4.6 without).
+    const bool bounded = chunk > 4 * kSampleThreads;
     bool first = true;
     int g = v0 + 4 * (int)threadIdx.x;
     u32x4 next = {0u, 0u, 0u, 0u};
@@ -157,11 +168,15 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             xv[q] = widen_raw<T>(raw[q]);
-            lu[q] = __builtin_amdgcn_logf((float)(0x7fffffu - (c[q] >> 9)) + 0.5f);
-            up[q] = __builtin_fmaf(lu[q], -kLn2, 23.f * kLn2 + kBoundSlack) + y_upper(xv[q]);
+            lu[q] = 0.f;
+            up[q] = __builtin_inff();
+            if (bounded) {
+                lu[q] = __builtin_amdgcn_logf((float)(0x7fffffu - (c[q] >> 9)) + 0.5f);
+                up[q] = __builtin_fmaf(lu[q], -kLn2, 23.f * kLn2 + kBoundSlack) + y_upper(xv[q]);
+            }
             if constexpr (!VEC) up[q] = g + q < v1 ? up[q] : -__builtin_inff();
         }
-        if (first) {
+        if (first && bounded) {
             // a first threshold: -log(u) <= (1 - u) / u bounds the noise from below
             first = false;
             uint32_t low = 0u;
@@ -175,7 +190,14 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
                 const bool use = (xv[q] == xv[q]) & (lo == lo) & (VEC || g + q < v1);
                 low = use ? max(low, f32_order_key(lo)) : low;
             }
-            atomicMax(&s_thr, low);
+            // the 16 lanes of each DPP row, then one lane of each: an LDS atomic of all 64
+            // lanes costs a round per lane (120 rows of 151936 bf16 logits 27.5 us, 23.7 so).
+            // A row whose last lane has no group adds nothing: a lower threshold.
+            low = max(low, row_shr<1>(low));
+            low = max(low, row_shr<2>(low));
+            low = max(low, row_shr<4>(low));
+            low = max(low, row_shr<8>(low));
+            if ((threadIdx.x & 15) == 15) atomicMax(&s_thr, low);
         }
         // candidates at or below the threshold cannot win (their exact value is
         // below their bound); it stays under +inf, so that equal infinities are
@@ -190,7 +212,7 @@ __global__ __launch_bounds__(kSampleThreads) void sample_rows_kernel(
                 // -inf is no candidate: not every such element is evaluated, and a row of
                 // nothing else gives id 0 without one
                 best = val != -__builtin_inff() && k > best ? k : best;
-                if (val == val) atomicMax(&s_thr, f32_order_key(val));
+                if (bounded && val == val) atomicMax(&s_thr, f32_order_key(val));
             }
         }
         if (!more) break;
