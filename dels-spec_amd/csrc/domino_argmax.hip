@@ -271,9 +271,7 @@ __global__ __launch_bounds__(kDomThreads) void domino_argmax_kernel(DominoArgs a
     if (u < units) consume(tr0, u);
     if (u + 2 < units) load_unit(u + 2, tr0);
     if (u + 1 < units) consume(tr1, u + 1);
-    if (u + 3 < units) load_unit(u + 3, tr1);
     if (u + 2 < units) consume(tr0, u + 2);
-    if (u + 3 < units) consume(tr1, u + 3);
 
     argmax_wg_finish<kDomWaves>(fin, best, bidx, m0, s_val, s_idx, s_last, nullptr);
 }

@@ -49,7 +49,6 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
     __shared__ unsigned long long s_rowmax[kRows];          // the step's maximum slot word of each row
     __shared__ float s_ab[2][kResidentMaxSteps];
     __shared__ int64_t s_ids[kRows];
-    __shared__ int s_flag;
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);

@@ -23,8 +23,9 @@
 //   * argmax: every wave contracts its resident tiles against the rank and
 //     combines s = fma(-beta, prior, fma(dot, alpha, base)) as every kernel of
 //     the path does (rr_tiles_best: 2.2 us of an 11.1 us step with a running
-//     (score, index) pair for each of a lane's four rows, 1.65 here; 8 rows); the workgroup publishes each row's best as one slot word (order(score)
-//     in the high half, ~index above two flag bits in the low half, so the
+//     (score, index) pair for each of a lane's four rows, 1.65 here; 8 rows); the
+//     workgroup publishes each row's best as one slot word (order(score) in the
+//     high half, ~index above two flag bits in the low half, so the
 //     larger word is the argmax with ties to the lower index) and every
 //     workgroup reads all nwg slots of each row, takes the maximum and so
 //     knows the step's ids for its GRU units.  Each workgroup owns its slots
@@ -342,7 +343,6 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
         if (r_pl.n <= 2 * kRrThreads) return rr_read_words<2>(a, rank_words, r_pl, tag, map);
         return rr_read_words<4>(a, rank_words, r_pl, tag, map);
     };
-
 
     // ---- prefix: h_0 = GRU(gi_table[prefix], 0) --------------------------------
     compute_gh(true);
