@@ -504,9 +504,14 @@ __global__ __launch_bounds__(kRrThreads) void rollout_resident_kernel(RrArgs a) 
             gru_publish(s_ids, 1, rr_tag(gen, s + 1));
             // the other workgroups read the state later than those that project the
             // rank from it: 8 MB of words (8 rows) on their way to everyone at once
-            // delay the ones that the step waits for (8 rows 10.45 -> 10.1 us a step,
-            // 24 rows 17.0 -> 16.2; half the pause gains nothing, more loses again)
-            if (!rank_wg) __builtin_amdgcn_s_sleep(RG == 1 ? 40 : 56);
+            // delay the ones that the step waits for.  14 steps at V = 151936 without
+            // and with the pause, G = 1024: 1 / 4 / 8 / 16 rows 160 / 153 / 165 / 203 ->
+            // 149 / 148 / 161 / 197 us, 17 / 24 / 32 rows 253 / 250 / 262 -> 243 / 242 /
+            // 251; G = 512: 1 / 8 / 16 rows 159 / 155 / 175 -> 145 / 152 / 173, likewise
+            // at V = 2000 to 100000 (half the pause gains nothing, more loses again).  Two
+            // groups at G = 512 have half the words: 206 / 206 / 213 without, 211 / 209 /
+            // 218 with, so they take none.
+            if (!rank_wg && (RG == 1 || a.upw > 4)) __builtin_amdgcn_s_sleep(RG == 1 ? 40 : 56);
             ok = read_state(rr_tag(gen, s + 1));
         }
     }
