@@ -165,6 +165,11 @@ __global__ __launch_bounds__(kRrThreads) void markov_resident_kernel(MarkovRollo
             const unsigned long long key = rr_tiles_best<KS, BaseT, PriorT, VEC>(
                 bt, ltile, lds_tile, &s_rank[(16 * g + lcol) * kPitch + lkg * 8], braw[g], s_prior, T0, ntl, wave, lkg,
                 V, s_ab[0][s], s_ab[1][s]);
+            // Sixteen idle cycles.  Without them rollouts of 2 to 4 rows take 1.5 % longer (14
+            // steps, V = 151936, r = 256: 94.0 / 94.7 / 96.1 us for 2 / 3 / 4 rows, 93.4 / 93.7 /
+            // 95.1 with them; 1, 5, 8 and 16 rows the same): where the code or the polls fall,
+            // not what they do, makes the difference.
+            asm volatile("s_nop 7\n\ts_nop 7");
             if (kg == 0) s_key[wave][16 * g + col] = key;
         }
         __syncthreads();
