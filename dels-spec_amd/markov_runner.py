@@ -6,8 +6,10 @@ called at code/dflash.py:540-545): same keyword arguments, ``ValueError``
 checks and messages, ``__call__(prev_token_ids, base_logits) -> int64[B,
 steps]`` returning a fresh tensor, and ``_can_triton_fuse`` (true: the fused
 native path is active).  Each step's rank is the previous token's row of the
-merged embedding, gathered by the argmax kernel's own rank load, so a step is
-one launch; the ``steps`` launches are captured once by the C ABI
+merged embedding, gathered where the argmax reads it, so no launch writes a
+rank.  The rollout is one launch that holds the low-rank head on chip, with one
+behind it that stands in when it cannot have the whole GPU, or a launch per step
+where that is the faster route; either is captured once by the C ABI
 (``dels_markov_graph_create``) and replayed per call.
 """
 
