@@ -10,11 +10,11 @@
 // quantised rank of all rows lies in LDS in operand order (RG * r * 16 bytes:
 // 32 KiB for 64 rows at r = 512); a tile is half of the bf16 kernel's registers,
 // so three of them per wave are in flight at two waves per SIMD.  The GEMV
-// kernel that this replaces reads B once per 16 rows.  r = 512, V = 151936, bf16
-// base logits: 24 rows 23.8 -> 21.1 us, 40 rows 62.9 -> 26.6; V = 32000, 40 rows
-// 20.1 -> 14.5; r = 256, V = 65536, 40 / 63 rows 16.4 / 18.7 -> 14.8 / 15.5, and
-// V = 32000, 40 rows 12.3 -> 12.8, the one size measured that gained nothing;
-// 200 rows of an unaligned vocabulary of 50257, 74.6 -> 58.6.  (Above 63
+// kernel reads B once per 16 rows and keeps the sizes where that costs little
+// (rows8_eligible).  r = 512, V = 151936, bf16 base logits: 24 rows 23.8 -> 20.3 us,
+// 40 rows 60.5 -> 25.2; V = 32000, 40 rows 20.3 -> 14.8; r = 256, V = 65536, 40 / 63
+// rows 16.5 / 18.6 -> 14.4 / 15.0; 200 rows of an unaligned vocabulary of 50257, r =
+// 512, 73.0 -> 28.0.  (Above 63
 // rows aligned rows go to the tiled kernel: 96 rows 30 us there, 41 in a variant
 // of this one with eight groups.)
 #pragma once
